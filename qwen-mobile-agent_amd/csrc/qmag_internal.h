@@ -77,6 +77,11 @@ int launch_q8k_quant(const float *x, int nblocks, int8_t *xq, float *xd, int16_t
                      hipStream_t s);
 int launch_matvec(const int8_t *xq, const float *xd, const int16_t *xsum, const void *W,
                   int n_in, int n_out, int T, int wtype, float *out, hipStream_t s);
+// several tokens on the matrix cores (qmag_mm.hip); arguments as
+// launch_matvec's, checked there; mm_supported: the calls that take it
+bool mm_supported(int nb, int T, int wtype, const void *W);
+int launch_mm(const int8_t *xq, const float *xd, const int16_t *xsum, const void *W, int nb, int n_out, int T,
+              int wtype, float *out, hipStream_t s);
 // T = 1 with x in f32: the matvec quantises x to Q8_K itself (bit-identical);
 // available for the row lengths matvec_x_supported() accepts
 bool matvec_x_supported(int n_in);

@@ -12,7 +12,8 @@
 // Also here: Q6_K rows repacked into aligned planes (QMAG_TYPE_Q6_K_R, same
 // bytes and results, for large matrices such as the LM head), and one launch
 // for several matrices over the same x (the projections of one activation
-// vector), bit-identical to separate calls.
+// vector), bit-identical to separate calls.  Calls of several tokens go to the
+// matrix cores (qmag_mm.hip) where that is faster; launch_matvec decides.
 #include "qmag_internal.h"
 
 // Launch shape of the tiled matvec: wave steps of rows in flight per wave,
@@ -554,14 +555,15 @@ int launch_matvec(const int8_t *xq, const float *xd, const int16_t *xsum, const 
         return fail(QMAG_ERR_ARG, "matvec: n_in=%d n_out=%d T=%d", n_in, n_out, T);
     if (!xq || !xd || !W || !out || (wtype == QMAG_TYPE_Q4_K && !xsum))
         return fail(QMAG_ERR_ARG, "matvec: null pointer");
+    if (wtype != QMAG_TYPE_Q4_K && wtype != QMAG_TYPE_Q6_K && wtype != QMAG_TYPE_Q6_K_R)
+        return fail(QMAG_ERR_ARG, "matvec: unsupported wtype %d", wtype);
+    if (wtype == QMAG_TYPE_Q6_K_R && (n_in % (8 * QK_K) || ((uintptr_t)W & 15)))
+        return fail(QMAG_ERR_ARG, "matvec: repacked Q6_K needs n_in %% 2048 == 0 and 16-byte aligned rows");
+    if (mm_supported(n_in / QK_K, T, wtype, W))
+        return launch_mm(xq, xd, xsum, W, n_in / QK_K, n_out, T, wtype, out, s);
     if (wtype == QMAG_TYPE_Q4_K) return launch_mv_t<QMAG_TYPE_Q4_K>(xq, xd, xsum, W, n_in, n_out, T, out, s, nullptr);
     if (wtype == QMAG_TYPE_Q6_K) return launch_mv_t<QMAG_TYPE_Q6_K>(xq, xd, xsum, W, n_in, n_out, T, out, s, nullptr);
-    if (wtype == QMAG_TYPE_Q6_K_R) {
-        if (n_in % (8 * QK_K) || ((uintptr_t)W & 15))
-            return fail(QMAG_ERR_ARG, "matvec: repacked Q6_K needs n_in %% 2048 == 0 and 16-byte aligned rows");
-        return launch_mv_t<QMAG_TYPE_Q6_K_R>(xq, xd, xsum, W, n_in, n_out, T, out, s, nullptr);
-    }
-    return fail(QMAG_ERR_ARG, "matvec: unsupported wtype %d", wtype);
+    return launch_mv_t<QMAG_TYPE_Q6_K_R>(xq, xd, xsum, W, n_in, n_out, T, out, s, nullptr);
 }
 
 bool matvec_x_supported(int n_in) { return n_in > 0 && n_in % QK_K == 0 && tiled_nb(n_in / QK_K); }

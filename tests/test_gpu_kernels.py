@@ -242,3 +242,46 @@ def test_synth_weights_deterministic_and_scaled(qm, orc, wtype):
     assert np.array_equal(ra, rb_)
     w = orc.dequant(ra, wtype, n)
     assert abs(w.std() - 0.02) < 0.002 and abs(w.mean()) < 0.002
+
+
+@pytest.mark.parametrize("wtype", [12, 14, 270])
+@pytest.mark.parametrize("n_in,n_out,T", [
+    # the split-K kernel: 1 to 4 tiles of 16 tokens, rows and tokens off a tile, fewer
+    # super-blocks than waves, several per wave, 4 waves (512 workgroups) and 8
+    (2048, 1, 9), (256, 15, 16), (2048, 33, 17), (4096, 16, 48), (2048, 100, 49), (6144, 17, 65), (1280, 70, 130),
+    (256, 8200, 20),
+    # the tile kernel (64 and 112 tiles of 128 rows x 64 tokens upwards), one to three super-blocks
+    (2048, 2049, 449), (256, 1793, 513), (768, 1921, 450)])
+def test_matmul_several_tokens(qm, orc, wtype, n_in, n_out, T):
+    """The matrix-core kernels of the matmul seam against the oracle.  Their
+    integer block sums are exact; per super-block and output three fp32
+    roundings, then the sum over the super-blocks (and waves): (nb + 3) 2^-24
+    of the sum of the terms' magnitudes, which is below 4 sqrt(nb) max|y|
+    here."""
+    if wtype == 270 and n_in % 2048:
+        pytest.skip("repacked rows need n_in % 2048 == 0")
+    W = orc.quantize(orc.fill_normal(3 * n_in + n_out, n_in * n_out, 0.0, 0.02), 12 if wtype == 12 else 14)
+    x = orc.fill_normal(T, n_in * T, 0.0, 1.0)
+    Wd, xd, out = qm.DBuf.from_array(W), qm.DBuf.from_array(x), qm.DBuf(4 * T * n_out)
+    if wtype == 270:
+        qm.repack_q6k_dev(Wd, Wd, n_in, n_out)
+    qm.matmul_dev(xd, Wd, n_in, n_out, T, wtype, out)
+    got = out.download(np.float32).reshape(T, n_out)
+    ref = np.asarray(orc.matmul_q8k(x, W, n_in, n_out, T, 12 if wtype == 12 else 14)).reshape(T, n_out)
+    nb = n_in // 256
+    assert max_rel_err(got, ref) < (nb + 3) * 2.0 ** -24 * 4 * nb ** 0.5
+
+
+@pytest.mark.parametrize("off", [2, 4, 6])
+def test_matmul_several_tokens_row_offsets(qm, orc, off):
+    """Q6_K rows that start 2 or 4 bytes past a dword boundary: the one the
+    image path takes and the ones it leaves to the matvec kernels."""
+    n_in, n_out, T = 768, 50, 20
+    W = orc.quantize(orc.fill_normal(8, n_in * n_out, 0.0, 0.02), 14)
+    x = orc.fill_normal(9, n_in * T, 0.0, 1.0)
+    Wd, xd, out = qm.DBuf(W.nbytes + 16), qm.DBuf.from_array(x), qm.DBuf(4 * T * n_out)
+    Wd.upload(W, off)
+    qm.check(qm.lib().qmag_matmul_dev(xd.ptr, Wd.ptr + off, n_in, n_out, T, 14, out.ptr))
+    got = out.download(np.float32).reshape(T, n_out)
+    ref = np.asarray(orc.matmul_q8k(x, W, n_in, n_out, T, 14)).reshape(T, n_out)
+    assert max_rel_err(got, ref) < 6 * 2.0 ** -24 * 4 * 3 ** 0.5
