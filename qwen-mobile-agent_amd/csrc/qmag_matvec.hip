@@ -559,7 +559,7 @@ int launch_matvec(const int8_t *xq, const float *xd, const int16_t *xsum, const 
         return fail(QMAG_ERR_ARG, "matvec: unsupported wtype %d", wtype);
     if (wtype == QMAG_TYPE_Q6_K_R && (n_in % (8 * QK_K) || ((uintptr_t)W & 15)))
         return fail(QMAG_ERR_ARG, "matvec: repacked Q6_K needs n_in %% 2048 == 0 and 16-byte aligned rows");
-    if (mm_supported(n_in / QK_K, T, wtype, W))
+    if (mm_supported(n_in / QK_K, T, wtype))
         return launch_mm(xq, xd, xsum, W, n_in / QK_K, n_out, T, wtype, out, s);
     if (wtype == QMAG_TYPE_Q4_K) return launch_mv_t<QMAG_TYPE_Q4_K>(xq, xd, xsum, W, n_in, n_out, T, out, s, nullptr);
     if (wtype == QMAG_TYPE_Q6_K) return launch_mv_t<QMAG_TYPE_Q6_K>(xq, xd, xsum, W, n_in, n_out, T, out, s, nullptr);

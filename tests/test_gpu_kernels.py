@@ -274,8 +274,9 @@ def test_matmul_several_tokens(qm, orc, wtype, n_in, n_out, T):
 
 @pytest.mark.parametrize("off", [2, 4, 6])
 def test_matmul_several_tokens_row_offsets(qm, orc, off):
-    """Q6_K rows that start 2 or 4 bytes past a dword boundary: the one the
-    image path takes and the ones it leaves to the matvec kernels."""
+    """Q6_K rows that start 2, 4 or 6 bytes past a 16-byte boundary: the weight
+    image reads a block from the dword it starts in, by its offset in the
+    matrix."""
     n_in, n_out, T = 768, 50, 20
     W = orc.quantize(orc.fill_normal(8, n_in * n_out, 0.0, 0.02), 14)
     x = orc.fill_normal(9, n_in * T, 0.0, 1.0)
