@@ -227,8 +227,8 @@ struct ExpertRecs {
 };
 
 // --------------------------------------------------------------- gate/up --
-// A wave holds R = 32/LPR row pairs: lanes [0,32) the gate rows, lanes
-// [32,64) the matching up rows.  After the per-row reduction the two halves
+// grid: (row steps of all slots) x tokens.  A wave holds R = 32/LPR row pairs:
+// lanes [0,32) the gate rows, lanes [32,64) the matching up rows.  After the per-row reduction the two halves
 // swap values with permlane32 so the gate lane sees its up value.
 template <int NBE>
 __global__ __launch_bounds__(256) void gateup_kernel(const uint8_t *__restrict__ gate_exps,
@@ -256,6 +256,12 @@ __global__ __launch_bounds__(256) void gateup_kernel(const uint8_t *__restrict__
     const int slot = wave / steps_per_slot;
     if (slot > K) return;
     const int base = (wave % steps_per_slot) * R * U;
+    const int t = (int)blockIdx.y;
+    sel += (size_t)t * K;
+    xq += (size_t)t * NBE * QK_K;
+    xd += (size_t)t * NBE;
+    xs += (size_t)t * NBE * 16;
+    h += (size_t)t * (K + 1) * F;
 
     const uint8_t *mat;
     if (slot < K && recs.rec[0]) {
@@ -309,12 +315,17 @@ struct DownTask;
 template <>
 struct DownTask<QMAG_TYPE_Q4_K> {
     static constexpr int BLOCK = Q4K_BYTES;
-    __device__ static float dot(const uint8_t *blk, const int8_t *hq, const float *hd,
-                                const int16_t *hs, int ib, int q)
+    uint4 hdr, q0, q1;
+    __device__ void load(const uint8_t *blk, int q)
+    {
+        hdr = ld16(blk);
+        q0 = ld16(blk + 16 + 32 * q);
+        q1 = ld16(blk + 32 + 32 * q);
+    }
+    __device__ float dot(const int8_t *hq, const float *hd, const int16_t *hs, int ib, int q) const
     {
         Q4Act a;
         q4_load_act(a, hq, hd, hs, ib, q);
-        const uint4 hdr = ld16(blk), q0 = ld16(blk + 16 + 32 * q), q1 = ld16(blk + 32 + 32 * q);
         return q4_task(hdr, q0, q1, a, q);
     }
 };
@@ -322,18 +333,24 @@ struct DownTask<QMAG_TYPE_Q4_K> {
 template <>
 struct DownTask<QMAG_TYPE_Q6_K> {
     static constexpr int BLOCK = Q6K_BYTES;
-    __device__ static float dot(const uint8_t *blk, const int8_t *hq, const float *hd,
-                                const int16_t *, int ib, int q)
+    Q6Raw r;
+    __device__ void load(const uint8_t *blk, int q) { q6_load_raw(r, blk, q >> 1, q & 1); }
+    __device__ float dot(const int8_t *hq, const float *hd, const int16_t *, int ib, int q) const
     {
         Q6Act a;
         q6_load_act(a, hq, ib, q >> 1, q & 1);
-        Q6Raw r;
-        q6_load_raw(r, blk, q >> 1, q & 1);
         const int isum = group_sum_i<4>(q6_int_dot(r, a, q & 1));
         return q == 0 ? h2f(r.d) * hd[ib] * (float)isum : 0.0f;
     }
 };
 
+// grid: (rows / RPW) x tokens, four waves: wave w takes slots w, w + 4, w + 8
+// of the token (the shared expert is slot K), requests their rows at once, and
+// leaves its dots in LDS; then one thread per row adds them in the reference's
+// order.  One wave taking the nine slots in turn waited for each slot's rows;
+// with that, and a launch per token and stage, 5 tokens of n_embd 2048, n_ff
+// 512, 256 experts (Q4_K down) took 83 us a layer; now 31.  Latency bounds the
+// few tokens, then the reads (32 tokens: 576 MB a layer at 4.5 TB/s).
 template <int NBF, int TD, int TDS>
 __global__ __launch_bounds__(256) void down_kernel(const uint8_t *__restrict__ down_exps,
                                                    const uint8_t *__restrict__ down_sh, const ExpertRecs recs,
@@ -349,29 +366,45 @@ __global__ __launch_bounds__(256) void down_kernel(const uint8_t *__restrict__ d
     constexpr int LPR = TPR;                 // NBF in {1, 2, 4}
     constexpr int RPW = 64 / LPR;
     constexpr int F = NBF * QK_K;
-    const int lane = lane_id();
+    __shared__ float s_y[9][RPW];
+    const int lane = lane_id(), wv = (int)(threadIdx.x >> 6);
     const int sub = lane % LPR, rw = lane / LPR, q = sub & 3, ib = sub >> 2;
-    const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const int row = wave * RPW + rw;
-    if (wave * RPW >= N) return;               // wave-uniform
-    const int rowc = row < N ? row : N - 1;
+    const int rowc = min((int)blockIdx.x * RPW + rw, N - 1);
+    const int t = (int)blockIdx.y;
+    const size_t slot0 = (size_t)t * (K + 1), at = (size_t)rowc * NBF + ib;
+    sel += (size_t)t * K;
+    w += (size_t)t * K;
 
+    DownTask<TD> dt[2];                      // slots w, w + 4 (K <= 8)
+    DownTask<TDS> ds;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int k = wv + 4 * j;
+        if (k < K) {                         // wave-uniform
+            const uint8_t *mat = recs.rec[0] ? recs.rec[k] + 2 * recs.gu
+                                             : down_exps + (size_t)sel[k] * N * NBF * DownTask<TD>::BLOCK;
+            dt[j].load(mat + at * DownTask<TD>::BLOCK, q);
+        }
+    }
+    const bool shared = wv == (K & 3);
+    if (shared) ds.load(down_sh + at * DownTask<TDS>::BLOCK, q);
+    auto act = [&](int k, auto &task) __attribute__((always_inline)) {
+        const size_t s = slot0 + k;
+        const float d = group_sum<LPR>(task.dot(hq + s * F, hd + s * NBF, hs + s * (F / 16), ib, q));
+        if (sub == 0) s_y[k][rw] = d;
+    };
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+        if (wv + 4 * j < K) act(wv + 4 * j, dt[j]);
+    if (shared) act(K, ds);
+    __syncthreads();
+    const int row = (int)blockIdx.x * RPW + (int)threadIdx.x;
+    if ((int)threadIdx.x >= RPW || row >= N) return;
     float acc = 0.0f;
-    for (int k = 0; k < K; k++) {
-        const size_t slab = (size_t)N * NBF * DownTask<TD>::BLOCK;
-        const uint8_t *mat = recs.rec[0] ? recs.rec[k] + 2 * recs.gu : down_exps + (size_t)sel[k] * slab;
-        const uint8_t *blk = mat + ((size_t)rowc * NBF + ib) * DownTask<TD>::BLOCK;
-        const float d = group_sum<LPR>(DownTask<TD>::dot(blk, hq + (size_t)k * F, hd + (size_t)k * NBF,
-                                                         hs + (size_t)k * (F / 16), ib, q));
-        acc = __fadd_rn(acc, __fmul_rn(w[k], d));
-    }
-    {
-        const uint8_t *blk = down_sh + ((size_t)rowc * NBF + ib) * DownTask<TDS>::BLOCK;
-        const float d = group_sum<LPR>(DownTask<TDS>::dot(blk, hq + (size_t)K * F, hd + (size_t)K * NBF,
-                                                          hs + (size_t)K * (F / 16), ib, q));
-        acc = __fadd_rn(acc, __fmul_rn(gs[0], d));
-    }
-    if (sub == 0 && row < N) out[row] = resid ? __fadd_rn(acc, resid[row]) : acc;
+    for (int k = 0; k < K; k++) acc = __fadd_rn(acc, __fmul_rn(w[k], s_y[k][threadIdx.x]));
+    acc = __fadd_rn(acc, __fmul_rn(gs[t], s_y[K][threadIdx.x]));
+    const size_t o = (size_t)t * N + row;
+    out[o] = resid ? __fadd_rn(acc, resid[o]) : acc;
 }
 
 // ------------------------------------------------------------------ host --
@@ -482,10 +515,14 @@ static void launch_f32_down(const qmag_moe_layer *L, const int *sel, const float
 
 static bool pow2_in(int v, int lo, int hi) { return v >= lo && v <= hi && (v & (v - 1)) == 0; }
 
-// batches of at least this many tokens take the grouped expert GEMM
-// (qmag_prefill.hip) when QMAG_OPT_GROUPED is on; smaller ones the
-// per-token launch sequence below
-constexpr int GROUPED_MIN_T = 8;
+// Batches of at least this many tokens take the grouped expert GEMM
+// (qmag_prefill.hip) when QMAG_OPT_GROUPED is on; smaller ones the launch
+// sequence below, which reads an expert once per token that chose it but is
+// five short launches.  Grouped / sequence, us per layer, Q6_K down: n_embd
+// 2048, 256 experts, top 8: 8 tokens 66 / 50, 32 135 / 127, 64 168 / 223; 1024,
+// 64 experts, top 4: 32 44 / 39, 64 51 / 60; 4096, 128 experts, top 8: 16
+// 93 / 75, 32 107 / 116.
+constexpr int GROUPED_MIN_T = 36;
 
 int moe_check_layer(const qmag_moe_layer *L, bool need_exps)
 {
@@ -539,7 +576,8 @@ static MoeWs g_last;
 static int g_last_K = 0;
 
 template <int NBE>
-static void launch_gateup(const qmag_moe_layer *L, const MoeWs &ws, int t, const ExpertRecs &recs, hipStream_t s)
+static void launch_gateup(const qmag_moe_layer *L, const MoeWs &ws, int t, int nt, const ExpertRecs &recs,
+                          hipStream_t s)
 {
     constexpr int TPR = 4 * NBE;
     constexpr int LPR = TPR < 32 ? TPR : 32;
@@ -547,7 +585,7 @@ static void launch_gateup(const qmag_moe_layer *L, const MoeWs &ws, int t, const
     const int N = L->n_embd, F = L->n_ff, K = L->n_used, S = K + 1;
     const int steps = (F + R * 2 - 1) / (R * 2);
     const int waves = steps * S;
-    hipLaunchKernelGGL(gateup_kernel<NBE>, dim3((waves + 3) / 4), dim3(256), 0, s,
+    hipLaunchKernelGGL(gateup_kernel<NBE>, dim3((waves + 3) / 4, nt), dim3(256), 0, s,
                        (const uint8_t *)L->gate_exps, (const uint8_t *)L->up_exps,
                        (const uint8_t *)L->gate_shexp, (const uint8_t *)L->up_shexp, recs,
                        ws.sel + (size_t)t * K, K, F, ws.xq + (size_t)t * N, ws.xd + (size_t)t * (N / QK_K),
@@ -555,14 +593,12 @@ static void launch_gateup(const qmag_moe_layer *L, const MoeWs &ws, int t, const
 }
 
 template <int NBF, int TD, int TDS>
-static void launch_down3(const qmag_moe_layer *L, const MoeWs &ws, int t, const ExpertRecs &recs,
+static void launch_down3(const qmag_moe_layer *L, const MoeWs &ws, int t, int nt, const ExpertRecs &recs,
                          const float *resid, float *out, hipStream_t s)
 {
     const int N = L->n_embd, F = L->n_ff, K = L->n_used, S = K + 1;
     constexpr int RPW = 64 / (4 * NBF);
-    const int waves = (N + RPW - 1) / RPW;
-    // one wave per workgroup: the grid is only N/RPW waves, spread it over CUs
-    hipLaunchKernelGGL((down_kernel<NBF, TD, TDS>), dim3(waves), dim3(64), 0, s,
+    hipLaunchKernelGGL((down_kernel<NBF, TD, TDS>), dim3((N + RPW - 1) / RPW, nt), dim3(256), 0, s,
                        (const uint8_t *)L->down_exps, (const uint8_t *)L->down_shexp, recs,
                        ws.sel + (size_t)t * K, ws.w + (size_t)t * K, ws.gs + t, K, N,
                        ws.hq + (size_t)t * S * F, ws.hd + (size_t)t * S * (F / QK_K),
@@ -571,41 +607,41 @@ static void launch_down3(const qmag_moe_layer *L, const MoeWs &ws, int t, const 
 }
 
 template <int NBF>
-static void launch_down2(const qmag_moe_layer *L, const MoeWs &ws, int t, const ExpertRecs &recs,
+static void launch_down2(const qmag_moe_layer *L, const MoeWs &ws, int t, int nt, const ExpertRecs &recs,
                          const float *resid, float *out, hipStream_t s)
 {
     const bool r6 = L->t_down_exps == QMAG_TYPE_Q6_K, s6 = L->t_down_shexp == QMAG_TYPE_Q6_K;
-    if (r6 && s6) launch_down3<NBF, QMAG_TYPE_Q6_K, QMAG_TYPE_Q6_K>(L, ws, t, recs, resid, out, s);
-    else if (r6) launch_down3<NBF, QMAG_TYPE_Q6_K, QMAG_TYPE_Q4_K>(L, ws, t, recs, resid, out, s);
-    else if (s6) launch_down3<NBF, QMAG_TYPE_Q4_K, QMAG_TYPE_Q6_K>(L, ws, t, recs, resid, out, s);
-    else launch_down3<NBF, QMAG_TYPE_Q4_K, QMAG_TYPE_Q4_K>(L, ws, t, recs, resid, out, s);
+    if (r6 && s6) launch_down3<NBF, QMAG_TYPE_Q6_K, QMAG_TYPE_Q6_K>(L, ws, t, nt, recs, resid, out, s);
+    else if (r6) launch_down3<NBF, QMAG_TYPE_Q6_K, QMAG_TYPE_Q4_K>(L, ws, t, nt, recs, resid, out, s);
+    else if (s6) launch_down3<NBF, QMAG_TYPE_Q4_K, QMAG_TYPE_Q6_K>(L, ws, t, nt, recs, resid, out, s);
+    else launch_down3<NBF, QMAG_TYPE_Q4_K, QMAG_TYPE_Q4_K>(L, ws, t, nt, recs, resid, out, s);
 }
 
-// the per-token expert stages of the launch sequence: gate/up, Q8_K(h),
-// down + combine
-static int token_experts(const qmag_moe_layer *L, const MoeWs &ws, int t, const ExpertRecs &recs,
+// the expert stages of the launch sequence for tokens t .. t + nt - 1 (nt <=
+// 65,535; with expert records one token): gate/up, Q8_K(h), down + combine
+static int token_experts(const qmag_moe_layer *L, const MoeWs &ws, int t, int nt, const ExpertRecs &recs,
                          const float *resid, float *out, hipStream_t s)
 {
     const int N = L->n_embd, F = L->n_ff, K = L->n_used, S = K + 1;
     prof_begin(PROF_GATEUP, s);
     switch (N / QK_K) {
-    case 1: launch_gateup<1>(L, ws, t, recs, s); break;
-    case 2: launch_gateup<2>(L, ws, t, recs, s); break;
-    case 4: launch_gateup<4>(L, ws, t, recs, s); break;
-    case 8: launch_gateup<8>(L, ws, t, recs, s); break;
-    default: launch_gateup<16>(L, ws, t, recs, s); break;
+    case 1: launch_gateup<1>(L, ws, t, nt, recs, s); break;
+    case 2: launch_gateup<2>(L, ws, t, nt, recs, s); break;
+    case 4: launch_gateup<4>(L, ws, t, nt, recs, s); break;
+    case 8: launch_gateup<8>(L, ws, t, nt, recs, s); break;
+    default: launch_gateup<16>(L, ws, t, nt, recs, s); break;
     }
     prof_end(PROF_GATEUP, s);
     prof_begin(PROF_HQUANT, s);
-    int st = launch_q8k_quant(ws.h + (size_t)t * S * F, S * (F / QK_K), ws.hq + (size_t)t * S * F,
+    int st = launch_q8k_quant(ws.h + (size_t)t * S * F, nt * S * (F / QK_K), ws.hq + (size_t)t * S * F,
                               ws.hd + (size_t)t * S * (F / QK_K), ws.hs + (size_t)t * S * (F / 16), s);
     prof_end(PROF_HQUANT, s);
     if (st) return st;
     prof_begin(PROF_DOWN, s);
     switch (F / QK_K) {
-    case 1: launch_down2<1>(L, ws, t, recs, resid, out, s); break;
-    case 2: launch_down2<2>(L, ws, t, recs, resid, out, s); break;
-    default: launch_down2<4>(L, ws, t, recs, resid, out, s); break;
+    case 1: launch_down2<1>(L, ws, t, nt, recs, resid, out, s); break;
+    case 2: launch_down2<2>(L, ws, t, nt, recs, resid, out, s); break;
+    default: launch_down2<4>(L, ws, t, nt, recs, resid, out, s); break;
     }
     prof_end(PROF_DOWN, s);
     return QMAG_OK;
@@ -656,8 +692,9 @@ int moe_ffn(const qmag_moe_layer *L, const float *x, float *out, int T, const fl
         return QMAG_OK;
     }
     const ExpertRecs slabs = {};
-    for (int t = 0; t < T; t++) {
-        st = token_experts(L, ws, t, slabs, resid, out, s);
+    constexpr int STEP = 32768;                // tokens per launch (a grid dimension)
+    for (int t = 0; t < T; t += STEP) {
+        st = token_experts(L, ws, t, T - t < STEP ? T - t : STEP, slabs, resid, out, s);
         if (st) return st;
     }
     QMAG_HIP(hipGetLastError());
@@ -836,7 +873,7 @@ extern "C" int qmag_moe_ffn_paged_dev(const qmag_moe_layer *L, qmag_ecache *c, i
                             sel[(size_t)t * K + k]);
             }
         }
-        st = token_experts(L, ws, t, recs, nullptr, out, s);
+        st = token_experts(L, ws, t, 1, recs, nullptr, out, s);
         qmag_ecache_release(c);      // after the launches: later copies wait for them
         if (st) return st;
     }

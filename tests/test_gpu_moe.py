@@ -982,3 +982,39 @@ def test_grouped_prefill_random_large_batches(qm, orc):
                 acc = (acc + (np.float32(scale) * y).astype(np.float32)).astype(np.float32)
             assert max_rel_err(got[t], acc) < TOL, (case, t)
         rl.close()
+
+
+@pytest.mark.parametrize("t_down,t_down_sh", [(14, 12), (12, 14)])
+@pytest.mark.parametrize("T", [35, 36, 64, 65, 97])
+def test_moe_batch_chunk_edges(qm, orc, T, t_down, t_down_sh):
+    """Every expert chosen by every token (8 of 8), so each bucket holds T
+    pairs: 35 tokens take the launch sequence (a grid over the tokens), 36
+    the grouped GEMM with chunks of 36 (two 32-pair tiles), then full chunks
+    of 64 and ones of 1 and 33 pairs behind a full one; both down types in
+    one layer."""
+    hl = make_host_layer(orc, seed=41, n_embd=256, n_ff=256, n_expert=8, n_used=8, t_down=t_down,
+                         t_down_sh=t_down_sh)
+    rl = qm.ResidentLayer.from_host(hl)
+    x = orc.fill_normal(900 + T, T * 256, 0.0, 1.0)
+    check_layer_staged(qm, orc, rl, hl, x, T)
+    rl.close()
+
+
+@pytest.mark.parametrize("grouped", [True, False])
+def test_moe_batch_route_exact_ties(qm, orc, grouped):
+    """The lowest index wins among exactly equal probabilities in the batch
+    paths too (36 tokens: the grouped GEMM, and with it off the sequence)."""
+    T, E, K, N = 36, 80, 8, 256
+    hl = make_host_layer(orc, seed=6, n_embd=N, n_ff=256, n_expert=E, n_used=K, router_bias_std=0.0)
+    hl.gate_inp[:] = 0.0
+    hl.router_bias[:] = 0.0
+    hl.router_bias[[5, 20, 33, 70]] = [4.0, 3.0, 2.0, 1.0]
+    rl = qm.ResidentLayer.from_host(hl)
+    qm.set_grouped(grouped)
+    try:
+        run_layer(qm, rl, orc.fill_normal(3, T * N, 0.0, 1.0), T)
+        st = qm.moe_last_stage(E, K, 256, n_tok=T)
+    finally:
+        qm.set_grouped(True)
+    assert st["sel"].tolist() == [[5, 20, 33, 70, 0, 1, 2, 3]] * T
+    rl.close()
