@@ -102,6 +102,10 @@ int launch_matvec_x(const float *x, const void *W, int n_in, int n_out, int wtyp
 int launch_dequant(const void *W, int wtype, long n, float *y, hipStream_t s);
 int launch_f32dot(const float *x, const void *W, int n_in, int n_out, int T, int wtype, float *out,
                   hipStream_t s);
+// the same for several tokens on the fp32 matrix cores (qmag_mmf.hip);
+// mmf_supported: the calls that take it
+bool mmf_supported(int nb, int n_out, int T, int wtype);
+int launch_mmf(const float *x, const void *W, int nb, int n_out, int T, int wtype, float *out, hipStream_t s);
 int moe_ffn(const qmag_moe_layer *L, const float *x, float *out, int T, const float *resid,
             hipStream_t s);
 // need_exps = false: the routed expert slabs may be null (paged experts)

@@ -79,7 +79,8 @@ int launch_dequant(const void *W, int wtype, long n, float *y, hipStream_t s)
 // ------------------------------------------------------ fp32 matvec ----
 // out[t][r] = sum_i deq(W[r])_i * x[t][i].  x of one token sits in LDS; a row
 // is split into 64-value tasks (f32_task) spread over LPR lanes, each lane
-// looping over its tasks.  Grid: (row chunks, T).  A launch covers nb
+// looping over its tasks.  Grid: (row chunks, T).  Larger products of several
+// tokens go to the matrix cores (qmag_mmf.hip).  A launch covers nb
 // super-blocks of each row: the whole row, or for rows longer than the LDS
 // chunk one chunk of it (x_stride and rb then give the full rows' strides).
 constexpr int F32_MAX_IN = 8192;
@@ -154,6 +155,7 @@ int launch_f32dot(const float *x, const void *W, int n_in, int n_out, int T, int
     if (!x || !W || !out) return fail(QMAG_ERR_ARG, "f32 matvec: null pointer");
     if (wtype != QMAG_TYPE_Q4_K && wtype != QMAG_TYPE_Q6_K)
         return fail(QMAG_ERR_ARG, "f32 matvec: unsupported wtype %d", wtype);
+    if (mmf_supported(n_in / QK_K, n_out, T, wtype)) return launch_mmf(x, W, n_in / QK_K, n_out, T, wtype, out, s);
     const size_t bb = wtype == QMAG_TYPE_Q4_K ? Q4K_BYTES : Q6K_BYTES, rb = (size_t)(n_in / QK_K) * bb;
     auto launch = [&](const float *xc, const uint8_t *wc, int nbc, float *o) {
         return wtype == QMAG_TYPE_Q4_K ? launch_f32dot_t<QMAG_TYPE_Q4_K>(xc, wc, nbc, n_out, T, o, s, n_in, rb)
