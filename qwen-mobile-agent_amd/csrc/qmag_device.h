@@ -426,15 +426,37 @@ __device__ __forceinline__ int q6_int_dot(const Q6Raw &r, const Q6Act &a, int l1
 // One 64-value task of an fp32 dot deq(row) . x (quants.c:80-133): Q4_K task
 // t covers the nibble group t & 3 of super-block t >> 2 (its 16-byte header
 // and 32 bytes of nibbles), Q6_K task t a quarter of super-block t >> 2.  xs
-// is the fp32 operand (in LDS).  The tasks of a row summed in any order give
-// the row's dot to fp32 rounding.
-template <int WT>
-__device__ __forceinline__ float f32_task(const uint8_t *row, int t, const float *xs)
+// is the fp32 operand, in LDS with 4 floats of padding after every 64
+// (f32_at): the lanes of a row read it 64 floats apart, which unpadded all
+// fall on the same four banks (2048 x 2048 Q4_K: 8 tokens 16.3 us, 5.8 padded;
+// a 12-token layer of n_embd 2048 97 us, 72 padded).  The tasks of a row summed in any order give the row's dot
+// to fp32 rounding.  load takes the task's bytes, so that a caller can request
+// several tasks before the first dot.
+__device__ __forceinline__ constexpr int f32_at(int i) { return i + 4 * (i >> 6); }
+constexpr int f32_padded(int n) { return n + n / 16; }
+// n floats (a multiple of 64) of src into the padded operand, by the workgroup
+__device__ __forceinline__ void f32_stage(float *xs, const float *src, int n)
 {
-    const int ib = t >> 2, q = t & 3;
-    if constexpr (WT == QMAG_TYPE_Q4_K) {
-        const uint8_t *b = row + (size_t)ib * Q4K_BYTES;
-        const uint4 hdr = ld16(b), q0 = ld16(b + 16 + 32 * q), q1 = ld16(b + 32 + 32 * q);
+    for (int i = (int)threadIdx.x; i < n / 4; i += (int)blockDim.x) ((float4 *)xs)[i + (i >> 4)] = ldg4(src + 4 * i);
+}
+template <int WT>
+struct F32Task;
+
+template <>
+struct F32Task<QMAG_TYPE_Q4_K> {
+    static constexpr int BLOCK = Q4K_BYTES;
+    uint4 hdr, q0, q1;
+    __device__ __forceinline__ void load(const uint8_t *row, int t)
+    {
+        const uint8_t *b = row + (size_t)(t >> 2) * Q4K_BYTES;
+        const int q = t & 3;
+        hdr = ld16(b);
+        q0 = ld16(b + 16 + 32 * q);
+        q1 = ld16(b + 32 + 32 * q);
+    }
+    __device__ __forceinline__ float dot(int t, const float *xs) const
+    {
+        const int q = t & 3;
         const float d = h2f(hdr.x & 0xffff), dmin = h2f(hdr.x >> 16);
         uint32_t s1, m1, s2, m2;
         q4_scale_min(2 * q, hdr.y, hdr.z, hdr.w, s1, m1);
@@ -442,7 +464,7 @@ __device__ __forceinline__ float f32_task(const uint8_t *row, int t, const float
         const float d1 = d * (float)s1, dm1 = dmin * (float)m1;
         const float d2 = d * (float)s2, dm2 = dmin * (float)m2;
         const uint32_t qw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-        const float4 *xv = (const float4 *)(xs + ib * QK_K + 64 * q);
+        const float4 *xv = (const float4 *)(xs + f32_at(64 * t));
         float lo = 0.0f, hi = 0.0f;
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -454,11 +476,20 @@ __device__ __forceinline__ float f32_task(const uint8_t *row, int t, const float
                   (d2 * (float)((w >> 20) & 15) - dm2) * c.z + (d2 * (float)((w >> 28) & 15) - dm2) * c.w;
         }
         return lo + hi;
-    } else {
-        const uint8_t *b = row + (size_t)ib * Q6K_BYTES;
-        const int n = q >> 1, l16 = q & 1;
-        Q6Raw r;
-        q6_load_raw(r, b, n, l16);
+    }
+};
+
+template <>
+struct F32Task<QMAG_TYPE_Q6_K> {
+    static constexpr int BLOCK = Q6K_BYTES;
+    Q6Raw r;
+    __device__ __forceinline__ void load(const uint8_t *row, int t)
+    {
+        q6_load_raw(r, row + (size_t)(t >> 2) * Q6K_BYTES, (t >> 1) & 1, t & 1);
+    }
+    __device__ __forceinline__ float dot(int t, const float *xs) const
+    {
+        const int ib = t >> 2, n = (t >> 1) & 1, l16 = t & 1;
         const float d = h2f(r.d);
         const uint64_t sc8 = ((uint64_t)r.sc.y << 32) | r.sc.x;
         const uint32_t L[4] = {r.ql_lo.x, r.ql_lo.y, r.ql_lo.z, r.ql_lo.w};
@@ -468,7 +499,7 @@ __device__ __forceinline__ float f32_task(const uint8_t *row, int t, const float
 #pragma unroll
         for (int Q = 0; Q < 4; Q++) {
             const float ds = d * (float)(int)(int8_t)((sc8 >> (8 * (l16 + 2 * Q))) & 255);
-            const float4 *xv = (const float4 *)(xs + ib * QK_K + 128 * n + 32 * Q + 16 * l16);
+            const float4 *xv = (const float4 *)(xs + f32_at(ib * QK_K + 128 * n + 32 * Q + 16 * l16));
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const uint32_t src = (Q & 1) ? H[k] : L[k];
@@ -481,6 +512,14 @@ __device__ __forceinline__ float f32_task(const uint8_t *row, int t, const float
         }
         return acc;
     }
+};
+
+template <int WT>
+__device__ __forceinline__ float f32_task(const uint8_t *row, int t, const float *xs)
+{
+    F32Task<WT> k;
+    k.load(row, t);
+    return k.dot(t, xs);
 }
 
 // ---------------------------------------------------------- routing ----

@@ -10,8 +10,8 @@
 // kept as accurate as the one-token kernel's lane tree: chains of 8 products
 // (two MFMAs), added pairwise within a super-block and over the waves (one
 // chain per step of 64 products gave 1.57e-7 of the result against 9.7e-8).
-// What bounds it at 24 tokens x 2048 x 2048 (44.4 -> 8.6 us with Q4_K rows,
-// 26.5 -> 9.6 with Q6_K) is the round trips of a wave's super-block; requesting
+// What bounds it at 24 tokens x 2048 x 2048 (8.6 us with Q4_K rows, 9.6 with
+// Q6_K; the one-token kernel 13.4 and 20.8) is the round trips of a wave's super-block; requesting
 // x a step ahead cost more in registers (two waves per SIMD) than it hid: 10.1.
 #include "qmag_mfma.h"
 
@@ -138,14 +138,15 @@ static int launch_mmf_t(const float *x, const uint8_t *W, int nb, int n_out, int
     return QMAG_OK;
 }
 
-// The one-token kernel spreads over the tokens and reads few rows faster; its
+// The one-token kernel spreads over the tokens and takes few rows faster; its
 // time grows with rows x tokens, this one's with a wave's super-blocks and
-// tiles.  Old / new, us: Q4_K 2048 x 2048 x 2 tokens 5.7 / 5.3, x 4 9.1 / 5.4;
-// n_in 4096, 100 rows x 48 11.2 / 16.9, 4096 rows x 2 17.1 / 8.8; Q6_K 2048 x
-// 2048 x 4 5.9 / 6.3, x 8 10.1 / 6.4; 4096, 4096 rows x 2 11.7 / 11.3.
+// tiles.  That kernel / this one, us: Q4_K 2048 x 2048 x 4 tokens 4.2 / 5.4, x
+// 8 5.8 / 5.5, x 24 13.4 / 8.6; n_in 4096, 100 rows x 48 5.0 / 16.9, 4096 rows
+// x 2 6.8 / 8.7, x 4 10.2 / 9.1; Q6_K 2048 x 2048 x 4 5.1 / 6.3, x 8 8.1 / 6.4;
+// 4096, 4096 rows x 2 9.5 / 11.3, x 4 14.1 / 11.5.
 bool mmf_supported(int nb, int n_out, int T, int wtype)
 {
-    const long least = wtype == QMAG_TYPE_Q4_K ? 8000 : 15000;
+    const long least = wtype == QMAG_TYPE_Q4_K ? 16000 : 12000;
     return T >= 2 && nb <= (1 << 18) && (long)n_out * T >= (T > 16 ? 2 : 1) * least;
 }
 

@@ -417,8 +417,11 @@ constexpr int F32_MAX_N = 4096, F32_MAX_SF = 9 * 1024;   // n_embd; (n_used + 1)
 
 // h[t][s][i] = silu(gate_i . x[t]) * (up_i . x[t]) for slot s (s < K: expert
 // sel[t][s]; s = K: the shared expert).  Grid (row blocks, K + 1, T); LPR
-// lanes per row.  Workgroup (0, K, t) also writes the fp32 shared gate
-// sigmoid(wsh . x[t]) (nn.c:477-479) to gs[t].
+// lanes per row, F32_U row steps per wave.  The first task of every row is
+// requested ahead of x (whose barrier it would otherwise wait behind), and the
+// two rows of a step read x from LDS together.  Workgroup (0, K, t) also
+// writes the fp32 shared gate sigmoid(wsh . x[t]) (nn.c:477-479) to gs[t].
+constexpr int F32_U = 2;
 template <int LPR>
 __global__ __launch_bounds__(256) void moe_f32_gateup_kernel(const uint8_t *__restrict__ gate_exps,
                                                              const uint8_t *__restrict__ up_exps,
@@ -429,29 +432,43 @@ __global__ __launch_bounds__(256) void moe_f32_gateup_kernel(const uint8_t *__re
                                                              const float *__restrict__ x, float *__restrict__ h,
                                                              float *__restrict__ gs)
 {
-    __shared__ __align__(16) float s_x[F32_MAX_N];
+    __shared__ __align__(16) float s_x[f32_padded(F32_MAX_N)];
+    using Task = F32Task<QMAG_TYPE_Q4_K>;
     const int t = (int)blockIdx.z, s = (int)blockIdx.y, S = K + 1;
-    for (int i = (int)threadIdx.x; i < N / 4; i += (int)blockDim.x)
-        ((float4 *)s_x)[i] = ldg4(x + (size_t)t * N + 4 * i);
-    __syncthreads();
     const int nb = N / QK_K, ntask = 4 * nb;
     const size_t rb = (size_t)nb * Q4K_BYTES, slab = (size_t)F * rb;
     const uint8_t *ge = s < K ? gate_exps + (size_t)sel[(size_t)t * K + s] * slab : gate_shexp;
     const uint8_t *ue = s < K ? up_exps + (size_t)sel[(size_t)t * K + s] * slab : up_shexp;
     const int lane = lane_id(), wave = (int)(threadIdx.x >> 6), sub = lane % LPR;
-    const int row = ((int)blockIdx.x * 4 + wave) * (64 / LPR) + lane / LPR;
-    float g = 0.0f, u = 0.0f;
-    if (row < F)
-        for (int tk = sub; tk < ntask; tk += LPR) {
-            g += f32_task<QMAG_TYPE_Q4_K>(ge + (size_t)row * rb, tk, s_x);
-            u += f32_task<QMAG_TYPE_Q4_K>(ue + (size_t)row * rb, tk, s_x);
+    const int row0 = ((int)blockIdx.x * 4 + wave) * F32_U * (64 / LPR) + lane / LPR;
+    Task tg[F32_U], tu[F32_U];
+#pragma unroll
+    for (int u = 0; u < F32_U; u++) {
+        const int row = min(row0 + u * (64 / LPR), F - 1), tk = min(sub, ntask - 1);
+        tg[u].load(ge + (size_t)row * rb, tk);
+        tu[u].load(ue + (size_t)row * rb, tk);
+    }
+    f32_stage(s_x, x + (size_t)t * N, N);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < F32_U; u++) {
+        const int row = row0 + u * (64 / LPR), rowc = min(row, F - 1);
+        float g = 0.0f, v = 0.0f;
+        if (sub < ntask) {
+            g = tg[u].dot(sub, s_x);
+            v = tu[u].dot(sub, s_x);
         }
-    g = group_sum<LPR>(g);
-    u = group_sum<LPR>(u);
-    if (sub == 0 && row < F) h[((size_t)t * S + s) * F + row] = (g / (1.0f + expf(-g))) * u;
+        for (int tk = sub + LPR; tk < ntask; tk += LPR) {
+            g += f32_task<QMAG_TYPE_Q4_K>(ge + (size_t)rowc * rb, tk, s_x);
+            v += f32_task<QMAG_TYPE_Q4_K>(ue + (size_t)rowc * rb, tk, s_x);
+        }
+        g = group_sum<LPR>(g);
+        v = group_sum<LPR>(v);
+        if (sub == 0 && row < F) h[((size_t)t * S + s) * F + row] = (g / (1.0f + expf(-g))) * v;
+    }
     if (blockIdx.x == 0 && s == K && wave == 0) {
         float v = 0.0f;
-        for (int i = lane; i < N; i += 64) v += wsh[i] * s_x[i];
+        for (int i = lane; i < N; i += 64) v += wsh[i] * s_x[f32_at(i)];
         v = group_sum<64>(v);
         if (lane == 0) gs[t] = 1.0f / (1.0f + expf(-v));
     }
@@ -468,30 +485,33 @@ __global__ __launch_bounds__(256) void moe_f32_down_kernel(const uint8_t *__rest
                                                            const float *__restrict__ gs, int K, int N, int F,
                                                            const float *__restrict__ h, float *__restrict__ out)
 {
-    __shared__ __align__(16) float s_h[F32_MAX_SF];
+    __shared__ __align__(16) float s_h[f32_padded(F32_MAX_SF)];
     const int t = (int)blockIdx.y, S = K + 1;
-    for (int i = (int)threadIdx.x; i < S * F / 4; i += (int)blockDim.x)
-        ((float4 *)s_h)[i] = ldg4(h + (size_t)t * S * F + 4 * i);
-    __syncthreads();
-    const int nb = F / QK_K, ntask = 4 * nb;
-    const size_t rb = (size_t)nb * (TD == QMAG_TYPE_Q6_K ? Q6K_BYTES : Q4K_BYTES), slab = (size_t)N * rb;
-    const size_t rbs = (size_t)nb * (TDS == QMAG_TYPE_Q6_K ? Q6K_BYTES : Q4K_BYTES);
+    const int nb = F / QK_K;                   // LPR = 4 nb: one task per lane and slot
+    const size_t rb = (size_t)nb * F32Task<TD>::BLOCK, slab = (size_t)N * rb;
+    const size_t rbs = (size_t)nb * F32Task<TDS>::BLOCK;
     const int lane = lane_id(), wave = (int)(threadIdx.x >> 6), sub = lane % LPR;
     const int row = ((int)blockIdx.x * 4 + wave) * (64 / LPR) + lane / LPR;
     const bool live = row < N;
+    const int rowc = live ? row : N - 1;
+    sel += (size_t)t * K;
+    w += (size_t)t * K;
+    // the next slot's rows are requested before the present slot's dot, the
+    // first one's and the shared expert's ahead of h
+    F32Task<TD> cur, nxt;
+    F32Task<TDS> sh;
+    cur.load(down_exps + (size_t)sel[0] * slab + (size_t)rowc * rb, sub);
+    sh.load(down_shexp + (size_t)rowc * rbs, sub);
+    f32_stage(s_h, h + (size_t)t * S * F, S * F);
+    __syncthreads();
     float acc = 0.0f;
     for (int k = 0; k < K; k++) {
-        const uint8_t *dr = down_exps + (size_t)sel[(size_t)t * K + k] * slab + (size_t)(live ? row : 0) * rb;
-        float y = 0.0f;
-        if (live)
-            for (int tk = sub; tk < ntask; tk += LPR) y += f32_task<TD>(dr, tk, s_h + k * F);
-        y = group_sum<LPR>(y);
-        acc = __fadd_rn(acc, __fmul_rn(w[(size_t)t * K + k], y));
+        nxt.load(down_exps + (size_t)sel[min(k + 1, K - 1)] * slab + (size_t)rowc * rb, sub);
+        const float y = group_sum<LPR>(cur.dot(sub, s_h + f32_at(k * F)));
+        acc = __fadd_rn(acc, __fmul_rn(w[k], y));
+        cur = nxt;
     }
-    float y = 0.0f;
-    if (live)
-        for (int tk = sub; tk < ntask; tk += LPR) y += f32_task<TDS>(down_shexp + (size_t)row * rbs, tk, s_h + K * F);
-    y = group_sum<LPR>(y);
+    const float y = group_sum<LPR>(sh.dot(sub, s_h + f32_at(K * F)));
     acc = __fadd_rn(acc, __fmul_rn(gs[t], y));
     if (sub == 0 && live) out[(size_t)t * N + row] = acc;
 }
@@ -903,12 +923,12 @@ extern "C" int qmag_moe_ffn_f32_dev(const qmag_moe_layer *L, const float *x, flo
     st = route_tokens(L, x, T, false, ws, s);
     if (st) return st;
     const int ntask = 4 * (N / QK_K);
-    const dim3 gu_grid((unsigned)((F + 15) / 16), (unsigned)S, (unsigned)T);
+    const dim3 gu_grid((unsigned)((F + 16 * F32_U - 1) / (16 * F32_U)), (unsigned)S, (unsigned)T);
     const uint8_t *ge = (const uint8_t *)L->gate_exps, *ue = (const uint8_t *)L->up_exps;
     const uint8_t *gsh = (const uint8_t *)L->gate_shexp, *ush = (const uint8_t *)L->up_shexp;
     prof_begin(PROF_GATEUP, s);
     if (ntask >= 32) {
-        hipLaunchKernelGGL(moe_f32_gateup_kernel<32>, dim3((F + 7) / 8, S, T), dim3(256), 0, s, ge, ue, gsh, ush,
+        hipLaunchKernelGGL(moe_f32_gateup_kernel<32>, dim3((F + 8 * F32_U - 1) / (8 * F32_U), S, T), dim3(256), 0, s, ge, ue, gsh, ush,
                            L->gate_inp_shexp, ws.sel, K, N, F, x, ws.h, ws.gs);
     } else {
         hipLaunchKernelGGL(moe_f32_gateup_kernel<16>, gu_grid, dim3(256), 0, s, ge, ue, gsh, ush, L->gate_inp_shexp,

@@ -90,12 +90,11 @@ __global__ __launch_bounds__(256) void f32dot_kernel(const uint8_t *__restrict__
                                                      float *__restrict__ out, int nb, int n_out, int x_stride,
                                                      size_t rb)
 {
-    __shared__ __align__(16) float s_x[F32_MAX_IN];
+    __shared__ __align__(16) float s_x[f32_padded(F32_MAX_IN)];
     const int t = (int)blockIdx.y;
     const int n_in = nb * QK_K;
     const float *xt = x + (size_t)t * x_stride;
-    for (int i = (int)threadIdx.x; i < n_in / 4; i += (int)blockDim.x)
-        ((float4 *)s_x)[i] = ldg4(xt + 4 * i);
+    f32_stage(s_x, xt, n_in);
     __syncthreads();
     const int lane = lane_id(), sub = lane % LPR;
     const int rows_per_wave = 64 / LPR;
