@@ -189,13 +189,14 @@ int qmag_q8k_quant_dev(const float *x, int n, int T, int8_t *xq, float *xd, int1
 
 /* out[t][r] = row_r(W) . Q8_K(x[t]) for pre-quantised activations;
    mm_worker, nn.c:276-289.  n_in: any multiple of 256 (powers of two up to
-   8192 run the tiled kernel, other lengths a kernel of one wave per row). */
+   8192 run the tiled kernel, other lengths a kernel of one wave per row;
+   several tokens run on the matrix cores, see qmag_mm.hip). */
 int qmag_matmul_q8k_dev(const int8_t *xq, const float *xd, const int16_t *xsum,
                         const void *W, int n_in, int n_out, int T, int wtype, float *out);
 
 /* matmul seam, nn.c:307-345: quantise each x[t] once, then the matvec (for
-   T = 1 and n_in a power of two up to 8192 a single launch: the matvec
-   quantises x itself, bit-identically).  n_in: any multiple of 256. */
+   T = 1 and n_in up to 32,768 a single launch: the matvec quantises x
+   itself, bit-identically).  n_in: any multiple of 256. */
 int qmag_matmul_dev(const float *x, const void *W, int n_in, int n_out, int T, int wtype,
                     float *out);
 

@@ -222,8 +222,7 @@ int launch_repack_q6k(const void *src, void *dst, int n_in, int n_out, hipStream
 // Q8_K of one activation vector of NB blocks into a workgroup's LDS: each
 // half-wave quantises one 256-block (8 values per lane, q8k_quant_half, the
 // same bits as q8k_quant_kernel), so a wave covers two blocks at once.
-template <int NB>
-__device__ __forceinline__ void q8k_x_to_lds(const float *__restrict__ xf, int8_t *s_xq, float *s_xd,
+__device__ __forceinline__ void q8k_x_to_lds(int NB, const float *__restrict__ xf, int8_t *s_xq, float *s_xd,
                                              int16_t *s_xs)
 {
     const int lane = lane_id(), wv = (int)(threadIdx.x >> 6), hl = lane >> 5, L = lane & 31;
@@ -288,7 +287,7 @@ __global__ __launch_bounds__(QMAG_MV_WG) void matvec_kernel(const uint8_t *__res
         __shared__ float s_xd[NB];
         __shared__ __align__(16) int16_t s_xs[N_IN / 16];
         load_rows(base0);                       // the weights are in flight during the quantisation
-        q8k_x_to_lds<NB>(xf, s_xq, s_xd, s_xs);
+        q8k_x_to_lds(NB, xf, s_xq, s_xd, s_xs);
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < TPL; j++) RT::load_act(act[j], s_xq, s_xd, s_xs, (sub + LPR * j) >> 2, q);
@@ -399,7 +398,7 @@ __global__ __launch_bounds__(QMAG_MV_WG) void matvec_group_kernel(MvGroup g, con
             }
         }
     }
-    q8k_x_to_lds<NB>(xf, s_xq, s_xd, s_xs);
+    q8k_x_to_lds(NB, xf, s_xq, s_xd, s_xs);
     __syncthreads();
     if (!live) return;
     float *out = g.out[m];
@@ -511,16 +510,73 @@ __global__ __launch_bounds__(256) void matvec_any_kernel(const uint8_t *__restri
     }
 }
 
+// The same at T = 1 with x in f32, one launch instead of two: every workgroup
+// requests its first row (up to 128 tasks, the rest in the loop), computes
+// Q8_K(x) into LDS as the tiled one-token kernel does, then runs the loop
+// above: the same bits.  Q6_K 5120 -> 1537: 5.5 us against 6.3, a launch of
+// about 2 us saved and Q8_K(x) computed beside the first rows' round trip.
+constexpr int MV_ANY_X_MAX_NB = 128;        // 37 KB of LDS
+template <int WT>
+__global__ __launch_bounds__(QMAG_MV_WG) void matvec_any_x_kernel(const uint8_t *__restrict__ W,
+                                                                  const float *__restrict__ xf,
+                                                                  float *__restrict__ out, int nb, int n_out)
+{
+    using RT = RowTask<WT>;
+    extern __shared__ __align__(16) uint8_t s_q8[];
+    int8_t *s_xq = (int8_t *)s_q8;
+    int16_t *s_xs = (int16_t *)(s_q8 + (size_t)nb * QK_K);
+    float *s_xd = (float *)(s_q8 + (size_t)nb * (QK_K + 32));
+    const int lane = lane_id(), q = lane & 3;
+    const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const int nwave = (int)((gridDim.x * blockDim.x) >> 6);
+    const size_t rb = (size_t)nb * RT::BLOCK;
+    const int ntask = 4 * nb;
+    typename RT::Raw first[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int tk = lane + 64 * j;
+        if (wave < n_out && tk < ntask) RT::load_raw(first[j], W + (size_t)wave * rb, tk >> 2, q, nb);
+        else first[j] = typename RT::Raw{};
+    }
+    q8k_x_to_lds(nb, xf, s_xq, s_xd, s_xs);
+    __syncthreads();
+    for (int row = wave; row < n_out; row += nwave) {
+        float v = 0.0f;
+        auto add = [&](const typename RT::Raw &r, int tk) __attribute__((always_inline)) {
+            typename RT::Act a;
+            RT::load_act(a, s_xq, s_xd, s_xs, tk >> 2, q);
+            v += RT::dot(r, a, q);
+        };
+        int tk = lane;
+        if (row == wave) {
+#pragma unroll
+            for (int j = 0; j < 2; j++, tk += 64)
+                if (tk < ntask) add(first[j], tk);
+        }
+        for (; tk < ntask; tk += 64) {
+            typename RT::Raw r;
+            RT::load_raw(r, W + (size_t)row * rb, tk >> 2, q, nb);
+            add(r, tk);
+        }
+        v = group_sum<64>(v);
+        if (lane == 0) out[row] = v;
+    }
+}
+
 template <int WT>
 static int launch_mv_any(const int8_t *xq, const float *xd, const int16_t *xsum, const void *W, int nb,
-                         int n_out, int T, float *out, hipStream_t s)
+                         int n_out, int T, float *out, hipStream_t s, const float *xf)
 {
     const long cap = (long)(ctx().n_cu > 0 ? ctx().n_cu : 256) * 32;    // waves
     const long waves = n_out < cap ? n_out : cap;
     const int wgs = (int)((waves + 3) / 4);
     prof_begin(PROF_MATVEC, s);
-    hipLaunchKernelGGL(matvec_any_kernel<WT>, dim3(wgs), dim3(256), 0, s, (const uint8_t *)W, xq, xd, xsum, out,
-                       nb, n_out, T);
+    if (xf)
+        hipLaunchKernelGGL(matvec_any_x_kernel<WT>, dim3(wgs), dim3(QMAG_MV_WG), (size_t)nb * (QK_K + 32 + 4), s,
+                           (const uint8_t *)W, xf, out, nb, n_out);
+    else
+        hipLaunchKernelGGL(matvec_any_kernel<WT>, dim3(wgs), dim3(256), 0, s, (const uint8_t *)W, xq, xd, xsum, out,
+                           nb, n_out, T);
     prof_end(PROF_MATVEC, s);
     QMAG_HIP(hipGetLastError());
     return QMAG_OK;
@@ -534,8 +590,7 @@ static int launch_mv_t(const int8_t *xq, const float *xd, const int16_t *xsum, c
                        int n_in, int n_out, int T, float *out, hipStream_t s, const float *xf)
 {
     if (!tiled_nb(n_in / QK_K)) {
-        if (xf) return fail(QMAG_ERR_ARG, "matvec: internal: fused Q8_K path needs a tiled row length");
-        return launch_mv_any<WT>(xq, xd, xsum, W, n_in / QK_K, n_out, T, out, s);
+        return launch_mv_any<WT>(xq, xd, xsum, W, n_in / QK_K, n_out, T, out, s, xf);
     }
     switch (n_in / QK_K) {
     case 1: return launch_mv_nb<WT, 1>(xq, xd, xsum, W, n_out, T, out, s, xf);
@@ -566,7 +621,10 @@ int launch_matvec(const int8_t *xq, const float *xd, const int16_t *xsum, const 
     return launch_mv_t<QMAG_TYPE_Q6_K_R>(xq, xd, xsum, W, n_in, n_out, T, out, s, nullptr);
 }
 
-bool matvec_x_supported(int n_in) { return n_in > 0 && n_in % QK_K == 0 && tiled_nb(n_in / QK_K); }
+bool matvec_x_supported(int n_in)
+{
+    return n_in > 0 && n_in % QK_K == 0 && (tiled_nb(n_in / QK_K) || n_in / QK_K <= MV_ANY_X_MAX_NB);
+}
 
 int launch_matvec_x(const float *x, const void *W, int n_in, int n_out, int wtype, float *out, hipStream_t s)
 {

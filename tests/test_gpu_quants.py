@@ -110,10 +110,28 @@ def test_q8k_dot_subnormal_scales(qm, orc):
 
 
 @pytest.mark.parametrize("wtype", [12, 14])
+@pytest.mark.parametrize("n_in,n_out", [(768, 1), (1280, 37), (2816, 1030), (5120, 9), (32512, 5), (33024, 3)])
+def test_matmul_one_launch_any_row_length(qm, orc, wtype, n_in, n_out):
+    """At T = 1 a row length that is no power of two runs as one launch too (up
+    to 32,768 values, beyond which Q8_K(x) is its own launch): the bits of the
+    two-step path."""
+    W = orc.quantize(orc.fill_normal(n_in + 7, n_in * n_out, 0.0, 0.02), wtype)
+    x = orc.fill_normal(n_in, n_in, 0.0, 1.0)
+    Wd, xb, out = qm.DBuf.from_array(W), qm.DBuf.from_array(x), qm.DBuf(4 * n_out)
+    qm.matmul_dev(xb, Wd, n_in, n_out, 1, wtype, out)
+    one = out.download(np.uint32)
+    xq, xd, xs = qm.DBuf(n_in), qm.DBuf(n_in // 64), qm.DBuf(n_in // 8)
+    qm.q8k_quant_dev(xb, n_in, 1, xq, xd, xs)
+    qm.matmul_q8k_dev(xq, xd, xs, Wd, n_in, n_out, 1, wtype, out)
+    assert np.array_equal(one, out.download(np.uint32))
+    assert max_rel_err(one.view(np.float32), orc.matmul_q8k(x, W, n_in, n_out, 1, wtype)[0]) < 1e-4
+
+
+@pytest.mark.parametrize("wtype", [12, 14])
 @pytest.mark.parametrize("n_in,n_out,T", [
     # from the rule's line upwards: one and two tiles of 16 tokens per workgroup, rows and
     # tokens off a tile, 1 to 8 waves with one and several super-blocks each, two token blocks
-    (256, 7501, 2), (512, 1001, 15), (768, 940, 16), (1280, 1777, 17), (2304, 937, 33), (8448, 625, 48)])
+    (256, 8001, 2), (512, 1067, 15), (768, 1001, 16), (1280, 1889, 17), (2304, 971, 33), (8448, 667, 48)])
 def test_matmul_f32_several_tokens(qm, orc, wtype, n_in, n_out, T):
     """The fp32 matrix-core kernel against float64 over the oracle's
     dequantised weights: fp32 weights (one rounding) and sums of at most 8
