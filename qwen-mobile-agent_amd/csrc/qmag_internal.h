@@ -47,6 +47,7 @@ enum WsSlot {
     WS_FLAGS,                       // kernel status / counters
     WS_GRP,                         // grouped prefill: bucket counts/offsets, pair permutation
     WS_Y,                           // grouped prefill: per-pair down outputs
+    WS_XMB,                         // grouped prefill: Q8_K(x) sub-block sums times the block scale
     WS_SAMP,                        // sampler: per-chunk candidates and the merged list
     WS_HOSTIO,                      // qmag_moe_ffn_host: the device copies of x and out
     WS_F32PART,                     // fp32 matmul rows longer than one LDS chunk: per-chunk partials
@@ -115,7 +116,7 @@ int moe_check_layer(const qmag_moe_layer *L, bool need_exps = true);
 // part[kc][T][E]: x . Wr^T over 256-wide k chunk kc (no bias)
 int launch_router_mfma(const qmag_moe_layer *L, const float *x, int T, float *part, hipStream_t s);
 int moe_grouped(const qmag_moe_layer *L, int T, const int *sel, const float *w, const float *gs,
-                const int8_t *xq, const float *xd, const int16_t *xs, float *h, int8_t *hq, float *hd,
+                const int8_t *xq, const float *xd, const float *xmb, float *h, int8_t *hq, float *hd,
                 int16_t *hs, const float *resid, float *out, hipStream_t s);
 
 // persistent single-launch decode (qmag_fused.hip)

@@ -1,6 +1,6 @@
 // qmag_mfma.h -- Q4_K / Q6_K rows x Q8_K activations on the int8 matrix cores:
 // the weight operands, the LDS image they are built from, and the 32-row x
-// 64-token product loop shared by the matmul and the grouped expert kernels.
+// 64-token product loop of the matmul.
 //
 // The sub-block scale is folded into the weight operand, as two int8 digits
 // of the product q * scale, so that one MFMA chain per digit runs over a
@@ -97,37 +97,19 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// TWO: the first half of the rows from one matrix, the second half from another
-template <int WT, int ROWS, bool TWO = false>
+template <int WT, int ROWS>
 struct WImage {
     static constexpr bool Q4 = WT == QMAG_TYPE_Q4_K, REP = WT == QMAG_TYPE_Q6_K_R;
     static constexpr int BLOCK = Q4 ? Q4K_BYTES : Q6K_BYTES, PIECES = Q4 ? 9 : 13;
     static constexpr int STRIDE = Q4 ? 144 : 240;      // 36 or 60 words: 16 rows' reads on distinct banks
     static constexpr int BYTES = ROWS * STRIDE, NP = ROWS * PIECES, WP = (NP + 63) / 64;
-    const uint8_t *base, *base2, *row;  // the wave's first row(s) (uniform), the lane's row lane % ROWS
+    const uint8_t *base, *row;          // the wave's first row (uniform), the lane's row lane % ROWS
     uint32_t at;                        // the first row's offset in the matrix (modulo 2^32)
     int nb, src[WP], dst[WP];
     uint4 v[WP];
     uint32_t tail;
     uint8_t *img;
 
-    // ROWS / 2 rows at A and as many at B
-    __device__ __forceinline__ void init2(uint8_t *lds, const uint8_t *A, const uint8_t *B, int nb_)
-    {
-        static_assert(TWO && Q4, "");
-        img = lds;
-        nb = nb_;
-        base = A;
-        base2 = B;
-        at = 0;
-        const int rb = nb * BLOCK;
-#pragma unroll
-        for (int k = 0; k < WP; k++) {
-            const int p = min(lane_id() + 64 * k, NP - 1), r = p / PIECES, j = p % PIECES;
-            dst[k] = r * STRIDE + 16 * j;
-            src[k] = (r % (ROWS / 2)) * rb + 16 * j;
-        }
-    }
     __device__ __forceinline__ void init(uint8_t *lds, const uint8_t *W, int row0, int n_out, int nb_)
     {
         img = lds;
@@ -152,9 +134,8 @@ struct WImage {
     __device__ __forceinline__ void request(int k, int ib)
     {
         const uint32_t step = REP ? ((lane_id() + 64 * k) % PIECES < 12 ? 64u : 16u) : (uint32_t)BLOCK;
-        const uint8_t *from = TWO && lane_id() + 64 * k >= NP / 2 ? base2 : base;
         const uint32_t o = (uint32_t)src[k] + (uint32_t)ib * step;
-        v[k] = ld16(from + (o - (uint32_t)lead(at + o)));
+        v[k] = ld16(base + (o - (uint32_t)lead(at + o)));
     }
     __device__ __forceinline__ void request_tail(int ib)
     {

@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void topk_kernel(float *__restrict__ logits, i
                                                    float *__restrict__ wout,
                                                    float *__restrict__ gs_out,
                                                    int8_t *__restrict__ xq, float *__restrict__ xd,
-                                                   int16_t *__restrict__ xs)
+                                                   int16_t *__restrict__ xs, float *__restrict__ xmb)
 {
     constexpr int MB = 4;                     // 256-blocks per wave (n_embd <= 4096)
     __shared__ float s_red[4];
@@ -134,6 +134,10 @@ __global__ __launch_bounds__(256) void topk_kernel(float *__restrict__ logits, i
             ((uint32_t *)(xq + (size_t)t * N + b * QK_K))[lane] = r.packed;
             if (lane == 0) xd[(size_t)t * NB + b] = r.d;
             if ((lane & 3) == 0) xs[(size_t)t * (N / 16) + b * 16 + (lane >> 2)] = (int16_t)r.gsum;
+            // the grouped prefill's Q4_K min-term operand: d * (sum of the
+            // 32 values of each sub-block), lanes 8j .. 8j+7 holding sub-block j
+            const int s32 = r.gsum + __shfl_xor(r.gsum, 4);
+            if (xmb && (lane & 7) == 0) xmb[(size_t)t * (N / 32) + b * 8 + (lane >> 3)] = r.d * (float)s32;
             const int8_t *q8 = (const int8_t *)&r.packed;
             g += gw[i].x * (float)q8[0] * r.d + gw[i].y * (float)q8[1] * r.d + gw[i].z * (float)q8[2] * r.d +
                  gw[i].w * (float)q8[3] * r.d;
@@ -538,11 +542,12 @@ static bool pow2_in(int v, int lo, int hi) { return v >= lo && v <= hi && (v & (
 // Batches of at least this many tokens take the grouped expert GEMM
 // (qmag_prefill.hip) when QMAG_OPT_GROUPED is on; smaller ones the launch
 // sequence below, which reads an expert once per token that chose it but is
-// five short launches.  Grouped / sequence, us per layer, Q6_K down: n_embd
-// 2048, 256 experts, top 8: 8 tokens 66 / 50, 32 135 / 127, 64 168 / 223; 1024,
-// 64 experts, top 4: 32 44 / 39, 64 51 / 60; 4096, 128 experts, top 8: 16
-// 93 / 75, 32 107 / 116.
-constexpr int GROUPED_MIN_T = 36;
+// five short launches.  Grouped / sequence, us per layer, with a router bias
+// (uneven experts, the grouped form's better case): n_embd 2048, 256 experts,
+// top 8, Q6_K down: 8 tokens 56 / 43, 12 62 / 56, 16 66 / 67, 24 74 / 88; Q4_K
+// down: 16 60 / 57, 24 66 / 74; 4096, 128 experts: 12 57 / 50, 16 60 / 59, 24
+// 71 / 75; 1024, 64 experts, top 4: 16 36 / 28, 35 40 / 40.
+constexpr int GROUPED_MIN_T = 16;
 
 int moe_check_layer(const qmag_moe_layer *L, bool need_exps)
 {
@@ -566,7 +571,7 @@ struct MoeWs {
     float *logits, *w, *gs, *h, *hd;
     int *sel;
     int8_t *xq, *hq;
-    float *xd;
+    float *xd, *xmb;
     int16_t *xs, *hs;
 };
 
@@ -584,6 +589,7 @@ static int moe_ws(const qmag_moe_layer *L, int T, MoeWs &ws)
     WS(xq, int8_t, WS_XQ, (size_t)T * N);
     WS(xd, float, WS_XD, (size_t)T * (N / QK_K));
     WS(xs, int16_t, WS_XS, (size_t)T * (N / 16));
+    WS(xmb, float, WS_XMB, (size_t)T * (N / 32));
     WS(h, float, WS_H, (size_t)T * S * F);
     WS(hq, int8_t, WS_HQ, (size_t)T * S * F);
     WS(hd, float, WS_HD, (size_t)T * S * (F / QK_K));
@@ -685,7 +691,7 @@ static int route_tokens(const qmag_moe_layer *L, const float *x, int T, bool gro
     // the grouped router leaves one partial per 256-wide k chunk and no bias
     hipLaunchKernelGGL(topk_kernel, dim3(T), dim3(256), 0, s, ws.logits, grouped ? N / 256 : 1, (size_t)T * E,
                        grouped ? L->router_bias : nullptr, x, L->gate_inp_shexp, N, E, K, ws.sel, ws.w, ws.gs,
-                       ws.xq, ws.xd, ws.xs);
+                       ws.xq, ws.xd, ws.xs, grouped ? ws.xmb : nullptr);
     prof_end(PROF_TOPK, s);
     return QMAG_OK;
 }
@@ -704,7 +710,7 @@ int moe_ffn(const qmag_moe_layer *L, const float *x, float *out, int T, const fl
     st = route_tokens(L, x, T, grouped, ws, s);
     if (st) return st;
     if (grouped) {
-        st = moe_grouped(L, T, ws.sel, ws.w, ws.gs, ws.xq, ws.xd, ws.xs, ws.h, ws.hq, ws.hd, ws.hs, resid, out,
+        st = moe_grouped(L, T, ws.sel, ws.w, ws.gs, ws.xq, ws.xd, ws.xmb, ws.h, ws.hq, ws.hd, ws.hs, resid, out,
                          s);
         if (st) return st;
         g_last = ws;

@@ -167,7 +167,7 @@ OPT_GROUPED = 4
 
 
 def set_grouped(on: bool) -> None:
-    """Batches of >= 36 tokens: the grouped int8-MFMA expert GEMM (default) or
+    """Batches of >= 16 tokens: the grouped int8-MFMA expert GEMM (default) or
     the launch sequence."""
     check(lib().qmag_set_option(OPT_GROUPED, 1 if on else 0))
 

@@ -985,13 +985,13 @@ def test_grouped_prefill_random_large_batches(qm, orc):
 
 
 @pytest.mark.parametrize("t_down,t_down_sh", [(14, 12), (12, 14)])
-@pytest.mark.parametrize("T", [35, 36, 64, 65, 97])
+@pytest.mark.parametrize("T", [15, 16, 64, 65, 97])
 def test_moe_batch_chunk_edges(qm, orc, T, t_down, t_down_sh):
     """Every expert chosen by every token (8 of 8), so each bucket holds T
-    pairs: 35 tokens take the launch sequence (a grid over the tokens), 36
-    the grouped GEMM with chunks of 36 (two 32-pair tiles), then full chunks
-    of 64 and ones of 1 and 33 pairs behind a full one; both down types in
-    one layer."""
+    pairs: 15 tokens take the launch sequence (a grid over the tokens), 16
+    the grouped GEMM with chunks of one 16-pair tile, then full chunks of 64
+    and ones of 1 and 33 pairs behind a full one; both down types in one
+    layer."""
     hl = make_host_layer(orc, seed=41, n_embd=256, n_ff=256, n_expert=8, n_used=8, t_down=t_down,
                          t_down_sh=t_down_sh)
     rl = qm.ResidentLayer.from_host(hl)
