@@ -222,9 +222,11 @@ int launch_repack_q6k(const void *src, void *dst, int n_in, int n_out, hipStream
 // Q8_K of one activation vector of NB blocks into a workgroup's LDS: each
 // half-wave quantises one 256-block (8 values per lane, q8k_quant_half, the
 // same bits as q8k_quant_kernel), so a wave covers two blocks at once.
-__device__ __forceinline__ void q8k_x_to_lds(int NB, const float *__restrict__ xf, int8_t *s_xq, float *s_xd,
-                                             int16_t *s_xs)
+template <int NBC>                              // 0: nb blocks, not a constant
+__device__ __forceinline__ void q8k_x_to_lds(const float *__restrict__ xf, int8_t *s_xq, float *s_xd,
+                                             int16_t *s_xs, int nb = 0)
 {
+    const int NB = NBC ? NBC : nb;
     const int lane = lane_id(), wv = (int)(threadIdx.x >> 6), hl = lane >> 5, L = lane & 31;
     for (int b0 = 2 * wv; b0 < NB; b0 += 2 * (QMAG_MV_WG / 64)) {
         const int b = b0 + hl;
@@ -287,7 +289,7 @@ __global__ __launch_bounds__(QMAG_MV_WG) void matvec_kernel(const uint8_t *__res
         __shared__ float s_xd[NB];
         __shared__ __align__(16) int16_t s_xs[N_IN / 16];
         load_rows(base0);                       // the weights are in flight during the quantisation
-        q8k_x_to_lds(NB, xf, s_xq, s_xd, s_xs);
+        q8k_x_to_lds<NB>(xf, s_xq, s_xd, s_xs);
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < TPL; j++) RT::load_act(act[j], s_xq, s_xd, s_xs, (sub + LPR * j) >> 2, q);
@@ -398,7 +400,7 @@ __global__ __launch_bounds__(QMAG_MV_WG) void matvec_group_kernel(MvGroup g, con
             }
         }
     }
-    q8k_x_to_lds(NB, xf, s_xq, s_xd, s_xs);
+    q8k_x_to_lds<NB>(xf, s_xq, s_xd, s_xs);
     __syncthreads();
     if (!live) return;
     float *out = g.out[m];
@@ -538,7 +540,7 @@ __global__ __launch_bounds__(QMAG_MV_WG) void matvec_any_x_kernel(const uint8_t 
         if (wave < n_out && tk < ntask) RT::load_raw(first[j], W + (size_t)wave * rb, tk >> 2, q, nb);
         else first[j] = typename RT::Raw{};
     }
-    q8k_x_to_lds(nb, xf, s_xq, s_xd, s_xs);
+    q8k_x_to_lds<0>(xf, s_xq, s_xd, s_xs, nb);
     __syncthreads();
     for (int row = wave; row < n_out; row += nwave) {
         float v = 0.0f;
@@ -621,15 +623,22 @@ int launch_matvec(const int8_t *xq, const float *xd, const int16_t *xsum, const 
     return launch_mv_t<QMAG_TYPE_Q6_K_R>(xq, xd, xsum, W, n_in, n_out, T, out, s, nullptr);
 }
 
-bool matvec_x_supported(int n_in)
+// x and out overlapping: the two-step path reads all of x first, so the row
+// lengths that took it before the one-launch form keep it
+bool matvec_x_supported(int n_in, int n_out, const float *x, const float *out)
 {
-    return n_in > 0 && n_in % QK_K == 0 && (tiled_nb(n_in / QK_K) || n_in / QK_K <= MV_ANY_X_MAX_NB);
+    if (n_in <= 0 || n_in % QK_K) return false;
+    if (tiled_nb(n_in / QK_K)) return true;
+    const uintptr_t xa = (uintptr_t)x, oa = (uintptr_t)out;
+    const bool apart = xa + sizeof(float) * (size_t)n_in <= oa ||
+                       oa + sizeof(float) * (size_t)(n_out > 0 ? n_out : 0) <= xa;
+    return n_in / QK_K <= MV_ANY_X_MAX_NB && apart;
 }
 
 int launch_matvec_x(const float *x, const void *W, int n_in, int n_out, int wtype, float *out, hipStream_t s)
 {
     if (n_in <= 0 || n_in % QK_K || n_out <= 0) return fail(QMAG_ERR_ARG, "matvec: n_in=%d n_out=%d", n_in, n_out);
-    if (!matvec_x_supported(n_in)) return fail(QMAG_ERR_ARG, "matvec: internal: n_in=%d has no fused Q8_K form", n_in);
+    if (!matvec_x_supported(n_in, n_out, x, out)) return fail(QMAG_ERR_ARG, "matvec: internal: n_in=%d has no fused Q8_K form", n_in);
     if (!x || !W || !out) return fail(QMAG_ERR_ARG, "matvec: null pointer");
     if (wtype == QMAG_TYPE_Q4_K)
         return launch_mv_t<QMAG_TYPE_Q4_K>(nullptr, nullptr, nullptr, W, n_in, n_out, 1, out, s, x);

@@ -124,6 +124,9 @@ def test_matmul_one_launch_any_row_length(qm, orc, wtype, n_in, n_out):
     qm.q8k_quant_dev(xb, n_in, 1, xq, xd, xs)
     qm.matmul_q8k_dev(xq, xd, xs, Wd, n_in, n_out, 1, wtype, out)
     assert np.array_equal(one, out.download(np.uint32))
+    if n_out <= n_in:                          # out on x itself: x is read whole first
+        qm.check(qm.lib().qmag_matmul_dev(xb.ptr, Wd.ptr, n_in, n_out, 1, wtype, xb.ptr))
+        assert np.array_equal(one, xb.download(np.uint32, n_out))
     assert max_rel_err(one.view(np.float32), orc.matmul_q8k(x, W, n_in, n_out, 1, wtype)[0]) < 1e-4
 
 
