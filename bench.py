@@ -1,6 +1,6 @@
-"""Benchmark: MoE FFN decode on one MI355X (BASELINE.json metric).
+"""Benchmark: MoE FFN decode on one MI355X.
 
-Workload: a 40-layer qwen35moe MoE FFN stack,
+Workload (C4): a 40-layer qwen35moe MoE FFN stack,
 all experts resident in HBM, decoding 256 tokens one after another at batch
 1.  Per layer: router f32 2048->256, softmax top-8 renormalised, 8 routed
 experts + 1 shared expert (gate/up 2048->512 Q4_K, down 512->2048 Q6_K),
@@ -53,7 +53,7 @@ METRIC = "MoE FFN decode tokens/s + achieved HBM GB/s (% of peak), Q4_K/Q6_K, 1 
 FUSED_TRAFFIC = {"bytes": 869.4e6, "profile": "profiles/moe_decode_kernel_c4_hbm_counters.md",
                  "sources": ["qwen-mobile-agent_amd/csrc/qmag_fused.hip", "qwen-mobile-agent_amd/csrc/qmag_device.h",
                              "qwen-mobile-agent_amd/csrc/qmag_internal.h"],
-                 "source_sha16": "4b9c5003ac8317ef"}
+                 "source_sha16": "225acdf186835b2a"}
 
 
 def fused_source_sha16():
