@@ -16,6 +16,7 @@
 #pragma once
 
 #include "qmag_internal.h"
+#include "qmag_wimage.h"
 
 namespace qmag {
 
@@ -86,7 +87,7 @@ struct Q4Scales {
 // request against 64).  A Q6_K block is therefore read from the dword it
 // starts in, 0 or 2 bytes ahead of it; its image starts as far in, and the
 // reader shifts (misaligned 16-byte LDS reads instead cost 8-10% of the tile
-// kernel).
+// kernel).  Every address is WImageMap's (qmag_wimage.h).
 
 // orders a wave's LDS accesses across its lanes (they execute in order; this
 // holds the compiler to it)
@@ -98,11 +99,9 @@ __device__ __forceinline__ void wave_lds_order()
 }
 
 template <int WT, int ROWS>
-struct WImage {
-    static constexpr bool Q4 = WT == QMAG_TYPE_Q4_K, REP = WT == QMAG_TYPE_Q6_K_R;
-    static constexpr int BLOCK = Q4 ? Q4K_BYTES : Q6K_BYTES, PIECES = Q4 ? 9 : 13;
-    static constexpr int STRIDE = Q4 ? 144 : 240;      // 36 or 60 words: 16 rows' reads on distinct banks
-    static constexpr int BYTES = ROWS * STRIDE, NP = ROWS * PIECES, WP = (NP + 63) / 64;
+struct WImage : WImageMap<WT, ROWS> {
+    using M = WImageMap<WT, ROWS>;
+    using M::BLOCK, M::BYTES, M::lead, M::NP, M::PIECES, M::Q4, M::REP, M::STRIDE, M::WP;
     const uint8_t *base, *row;          // the wave's first row (uniform), the lane's row lane % ROWS
     uint32_t at;                        // the first row's offset in the matrix (modulo 2^32)
     int nb, src[WP], dst[WP];
@@ -114,37 +113,29 @@ struct WImage {
     {
         img = lds;
         nb = nb_;
-        const int first = min(row0, n_out - 1), rb = nb * BLOCK;
+        const int first = M::row(0, row0, n_out), rb = nb * BLOCK;
         base = W + (size_t)first * rb;
         at = (uint32_t)first * (uint32_t)rb;
-        row = base + (min(row0 + lane_id() % ROWS, n_out - 1) - first) * rb;
+        row = base + M::row_off(lane_id() % ROWS, row0, n_out, rb);
 #pragma unroll
         for (int k = 0; k < WP; k++) {
-            const int p = min(lane_id() + 64 * k, NP - 1), r = p / PIECES, j = p % PIECES;
-            const int rel = (min(row0 + r, n_out - 1) - first) * rb;
-            dst[k] = r * STRIDE + 16 * j;
-            if constexpr (!REP) src[k] = rel + 16 * j;
-            else if (j < 8) src[k] = rel + 64 * nb * ((j >> 1) & 1) + 16 * (2 * (j >> 2) + (j & 1));
-            else src[k] = rel + (j < 12 ? 128 * nb + 16 * (j - 8) : 192 * nb);
+            const int p = M::piece(lane_id(), k), r = p / PIECES, j = p % PIECES;
+            const int rel = M::row_off(r, row0, n_out, rb);
+            dst[k] = M::dst(r, j);
+            src[k] = rel + M::src(j, nb);
         }
     }
-    // bytes between the dword a block starts in and the block, by its offset
-    // in the matrix (so that no read starts ahead of it)
-    __device__ static __forceinline__ int lead(uint32_t off) { return WT == QMAG_TYPE_Q6_K ? (int)(off & 2) : 0; }
     __device__ __forceinline__ void request(int k, int ib)
     {
-        const uint32_t step = REP ? ((lane_id() + 64 * k) % PIECES < 12 ? 64u : 16u) : (uint32_t)BLOCK;
-        const uint32_t o = (uint32_t)src[k] + (uint32_t)ib * step;
+        const uint32_t o = (uint32_t)src[k] + (uint32_t)ib * M::step(M::piece(lane_id(), k) % PIECES);
         v[k] = ld16(base + (o - (uint32_t)lead(at + o)));
     }
     __device__ __forceinline__ void request_tail(int ib)
     {
-        if constexpr (REP) {
-            tail = ld2(row + 208 * nb + 2 * ib);
-        } else if constexpr (!Q4) {
-            const uint8_t *blk = row + ib * BLOCK;
-            tail = ld2(blk + 208 - lead(at + (uint32_t)(row - base) + (uint32_t)ib * BLOCK)) | (ld2(blk + 208) << 16);
-        }
+        if constexpr (Q4) return;
+        const uint8_t *t = row + ib * M::tail_step() + M::tail0(nb);
+        if constexpr (REP) tail = ld2(t);
+        else tail = ld2(t - lead(at + (uint32_t)(row - base) + (uint32_t)ib * BLOCK)) | (ld2(t) << 16);
     }
     __device__ __forceinline__ void request_all(int ib)
     {
