@@ -154,7 +154,13 @@ int launch_f32dot(const float *x, const void *W, int n_in, int n_out, int T, int
     if (!x || !W || !out) return fail(QMAG_ERR_ARG, "f32 matvec: null pointer");
     if (wtype != QMAG_TYPE_Q4_K && wtype != QMAG_TYPE_Q6_K)
         return fail(QMAG_ERR_ARG, "f32 matvec: unsupported wtype %d", wtype);
-    if (mmf_supported(n_in / QK_K, n_out, T, wtype)) return launch_mmf(x, W, n_in / QK_K, n_out, T, wtype, out, s);
+    // out may lie on x where the rows are longer than one LDS chunk: there the
+    // chunks' partials are written out only after all of x has been read, while
+    // the matrix-core kernel writes out as it reads
+    const uintptr_t xa = (uintptr_t)x, oa = (uintptr_t)out;
+    const bool apart = xa + sizeof(float) * (size_t)T * n_in <= oa || oa + sizeof(float) * (size_t)T * n_out <= xa;
+    if (mmf_supported(n_in / QK_K, n_out, T, wtype) && (apart || n_in <= F32_MAX_IN))
+        return launch_mmf(x, W, n_in / QK_K, n_out, T, wtype, out, s);
     const size_t bb = wtype == QMAG_TYPE_Q4_K ? Q4K_BYTES : Q6K_BYTES, rb = (size_t)(n_in / QK_K) * bb;
     auto launch = [&](const float *xc, const uint8_t *wc, int nbc, float *o) {
         return wtype == QMAG_TYPE_Q4_K ? launch_f32dot_t<QMAG_TYPE_Q4_K>(xc, wc, nbc, n_out, T, o, s, n_in, rb)

@@ -152,6 +152,26 @@ def test_matmul_f32_several_tokens(qm, orc, wtype, n_in, n_out, T):
 
 
 @pytest.mark.parametrize("wtype", [12, 14])
+@pytest.mark.parametrize("at", [0, 8448, 130000])
+def test_matmul_f32_out_on_x(qm, orc, wtype, at):
+    """Rows longer than one 8192-value chunk, several tokens, out on x (from
+    its float `at`; the last reaches past its end): the call reads all of x
+    first.  Each chunk is a sum of at most 128 products per lane, a lane tree
+    and one addition per chunk: far below 1e-4 of max|y|, while a token read
+    after it was overwritten gives wrong values throughout."""
+    n_in, n_out, T = 8448, 1003, 16
+    W = _rand_blocks(np.random.default_rng(77), wtype, n_in * n_out // 256)
+    x = orc.fill_normal(78, n_in * T, 0.0, 1.0)
+    buf = qm.DBuf(4 * (max(n_in * T, at + n_out * T)))
+    buf.upload(x)
+    Wd = qm.DBuf.from_array(W)
+    qm.check(qm.lib().qmag_matmul_f32_dev(buf.ptr, Wd.ptr, n_in, n_out, T, wtype, buf.ptr + 4 * at))
+    got = buf.download(np.float32)[at:at + n_out * T].reshape(T, n_out)
+    deq = orc.dequant(W, wtype, n_in * n_out).astype(np.float64).reshape(n_out, n_in)
+    assert max_rel_err(got, x.astype(np.float64).reshape(T, n_in) @ deq.T) < TOL
+
+
+@pytest.mark.parametrize("wtype", [12, 14])
 @pytest.mark.parametrize("n_in,n_out,T", [(256, 100, 1), (2048, 512, 1), (512, 2048, 3), (8192, 64, 2),
                                           (768, 77, 1), (12288, 40, 3), (16640, 33, 2), (24576, 17, 1)])
 def test_matmul_f32_dev(qm, orc, wtype, n_in, n_out, T):
