@@ -296,6 +296,38 @@ __device__ __forceinline__ v4h sums_f16(uint2 s)
                (_Float16)(int16_t)(s.y >> 16)};
 }
 
+// ------------------------------------------------------------ split over K --
+// The partial results of a workgroup whose nw waves split the nb super-blocks,
+// in LDS as [waves][MT][4][64].  One running sum per wave rounds the more the
+// longer the row, so where a wave has more than `chain` super-blocks (a long
+// row) it adds its sums there after every chain of them: each kernel's chain is
+// as long as leaves the error against 64 bits at or below a lane tree's.
+__host__ __device__ __forceinline__ bool long_row(int nb, int nw, int chain) { return nb > chain * nw; }
+template <int MT>
+__device__ __forceinline__ void put_partials(float *s_part, int wv, float (&r)[MT][4], bool add)
+{
+    float *p = s_part + wv * MT * 256 + lane_id();
+    if (add)
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) r[m][i] += p[(4 * m + i) * 64];
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            p[(4 * m + i) * 64] = r[m][i];
+            r[m][i] = 0.0f;
+        }
+}
+// LDS bytes of such a workgroup: an image per wave, then the partials, in the
+// images' place unless the rows are long
+inline size_t split_lds(int nb, int nw, int chain, int mt, int image)
+{
+    const size_t part = sizeof(float) * 256 * (size_t)mt;
+    return (size_t)nw * (long_row(nb, nw, chain) ? part + image : part > (size_t)image ? part : image);
+}
+
 // ------------------------------------------------------------------- tiles --
 // A workgroup of four waves: wave w holds 32 weight rows, all four share up to
 // 32 NT activation rows (tokens).  Per super-block those go through registers
@@ -312,28 +344,35 @@ struct TileLds {
 
 // The Q8_K rows a thread stages: 16-byte piece tid % 16 of tokens tid / 16 +
 // 16 k, the scale of token tid, half of the 16 sums of token tid / 2; row(t):
-// the row index of the workgroup's token t.
+// the row of the workgroup's token t, counted from the arrays' uniform bases.
+// The offsets are 32-bit (64 rows of at most 2^26 values): as pointers they
+// cost registers that the Q6_K loop does not have.
 template <int NT>
 struct TileSrc {
-    const int8_t *x[2 * NT];
-    const float *d;
-    const int16_t *s;
+    const int8_t *xq;
+    const float *xd;
+    const int16_t *xs;
+    uint32_t x[2 * NT], d, s;
     template <class Row>
-    __device__ __forceinline__ void init(const int8_t *xq, const float *xd, const int16_t *xsum, int nb, Row row)
+    __device__ __forceinline__ void init(const int8_t *q, const float *scales, const int16_t *sums, int nb, Row row)
     {
-        const int tid = (int)threadIdx.x;
+        const uint32_t tid = threadIdx.x;
+        xq = q;
+        xd = scales;
+        xs = sums;
 #pragma unroll
-        for (int k = 0; k < 2 * NT; k++) x[k] = xq + (size_t)row((tid >> 4) + 16 * k) * nb * QK_K + 16 * (tid & 15);
-        d = xd + (size_t)row(tid & (32 * NT - 1)) * nb;
-        s = xsum ? xsum + (size_t)row((tid & (64 * NT - 1)) >> 1) * nb * 16 + 8 * (tid & 1) : nullptr;
+        for (int k = 0; k < 2 * NT; k++) x[k] = (uint32_t)row((tid >> 4) + 16 * k) * (uint32_t)(nb * QK_K) + 16 * (tid & 15);
+        d = (uint32_t)row(tid & (32 * NT - 1)) * (uint32_t)nb;
+        s = (uint32_t)row((tid & (64 * NT - 1)) >> 1) * (uint32_t)(nb * 16) + 8 * (tid & 1);
     }
 };
 
 // r[m][i] of a lane: token 32 m + 8 (i / 4) + 4 (lane / 32) + i % 4, weight row
-// lane % 32.  LONG: the rows may have more than eight super-blocks.  The
-// image's block 0 has been requested.
+// lane % 32, over the super-blocks ib0 .. nb - 1 (ib0 a multiple of eight).  LONG:
+// these may be more than eight.  The image's block ib0 has been requested.
 template <int WT, int NT, bool LONG, class Img>
-__device__ __forceinline__ void tile_products(Img &img, int nb, const TileSrc<NT> &src, TileLds<NT> &lds, v16f (&r)[NT])
+__device__ __forceinline__ void tile_products(Img &img, int ib0, int nb, const TileSrc<NT> &src, TileLds<NT> &lds,
+                                              v16f (&r)[NT])
 {
     using Row = WRow<WT, 2>;
     const int tid = (int)threadIdx.x, lane = lane_id(), lr = lane & 31, h = lane >> 5;
@@ -343,9 +382,9 @@ __device__ __forceinline__ void tile_products(Img &img, int nb, const TileSrc<NT
     auto request = [&](int s, int ib, bool weights) __attribute__((always_inline)) {
         if (weights && s < Img::WP) img.request(s, ib);
         if (weights && s == 7) img.request_tail(ib);
-        if (s < 2 * NT) va[s] = ld16((const uint8_t *)src.x[s] + (size_t)ib * QK_K);
-        if (s == 5 && tid < 32 * NT) vd = ldg(src.d + ib);
-        if (Row::MIN && s == 6 && tid < 64 * NT) vs = ld16((const uint8_t *)(src.s + (size_t)ib * 16));
+        if (s < 2 * NT) va[s] = ld16((const uint8_t *)src.xq + (size_t)ib * QK_K + src.x[s]);
+        if (s == 5 && tid < 32 * NT) vd = ldg(src.xd + ib + src.d);
+        if (Row::MIN && s == 6 && tid < 64 * NT) vs = ld16((const uint8_t *)(src.xs + (size_t)ib * 16 + src.s));
     };
     auto stage = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -363,34 +402,19 @@ __device__ __forceinline__ void tile_products(Img &img, int nb, const TileSrc<NT
 #pragma unroll
         for (int i = 0; i < 16; i++) r[m][i] = tot[m][i] = 0.0f;
 #pragma unroll
-    for (int s = 0; s < 8; s++) request(s, 0, false);
+    for (int s = 0; s < 8; s++) request(s, ib0, false);
     img.store();
     stage(0);
     __syncthreads();
-    for (int ib = 0; ib < nb; ib++) {
+    for (int ib = ib0; ib < nb; ib++) {
         const int buf = ib & 1, nx = min(ib + 1, nb - 1);
         const Row w(img.block(), img.shift(ib));
         const int8_t *pa = lds.a[buf] + lr * TILE_ROW + 16 * h;
         v16i lo[NT], hi[NT];
-        v16f mn[NT];
 #pragma unroll
         for (int m = 0; m < NT; m++)
 #pragma unroll
             for (int i = 0; i < 16; i++) lo[m][i] = hi[m][i] = 0;
-        const float d = w.d();
-        float nm = 0.0f;
-        if constexpr (Row::MIN) {
-            nm = -w.dmin();
-            const v8h mb = w.mins8();
-#pragma unroll
-            for (int m = 0; m < NT; m++) {
-                v16f z;
-#pragma unroll
-                for (int i = 0; i < 16; i++) z[i] = 0.0f;
-                mn[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const v8h *)(lds.s[buf] + (32 * m + lr) * 16 + 8 * h),
-                                                               mb, z, 0, 0, 0);
-            }
-        }
         // Step by step: the next step's LDS reads, a share of the next
         // super-block's requests (all at once they hold the wave for the time
         // the address unit takes to accept them, 700-2,000 cycles), this
@@ -419,6 +443,23 @@ __device__ __forceinline__ void tile_products(Img &img, int nb, const TileSrc<NT
             if (s < 7) w.operands(raw, s + 1, bl[n], bh[n]);
             __builtin_amdgcn_sched_barrier(0);
         }
+        // the min term last: its 32 results would be as many registers through
+        // the steps
+        v16f mn[NT];
+        const float d = w.d();
+        float nm = 0.0f;
+        if constexpr (Row::MIN) {
+            nm = -w.dmin();
+            const v8h mb = w.mins8();
+#pragma unroll
+            for (int m = 0; m < NT; m++) {
+                v16f z;
+#pragma unroll
+                for (int i = 0; i < 16; i++) z[i] = 0.0f;
+                mn[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const v8h *)(lds.s[buf] + (32 * m + lr) * 16 + 8 * h),
+                                                               mb, z, 0, 0, 0);
+            }
+        }
 #pragma unroll
         for (int m = 0; m < NT; m++)
 #pragma unroll
@@ -433,11 +474,14 @@ __device__ __forceinline__ void tile_products(Img &img, int nb, const TileSrc<NT
                     r[m][i] = fmaf(xv[k], v, r[m][i]);
                 }
             }
-        if constexpr (LONG && !Row::MIN) {
+        if constexpr (LONG) {
             // sums of eight super-blocks are added up apart: one running sum
-            // over a long row would round more than the matvec's lane tree
-            // (Q6_K, n_in 8192: 1.07e-7 of the result against 7.4e-8)
-            if ((ib & 7) == 7)
+            // over a long row would round more than the matvec's lane tree (n_in
+            // 8192: Q6_K 1.07e-7 of the result against 7.4e-8; Q4_K weights of
+            // random bytes 1.04e-7 against 8.5e-8, now 7.5e-8).  With its
+            // registers Q4_K of 4096 values and more takes 3% longer where a CU
+            // has one workgroup (4096 x 4096 x 256 30.2 -> 31.1 us).
+            if ((ib & 7) == 7 && ib + 1 < nb)
 #pragma unroll
                 for (int m = 0; m < NT; m++) {
                     tot[m] += r[m];
@@ -449,7 +493,7 @@ __device__ __forceinline__ void tile_products(Img &img, int nb, const TileSrc<NT
         stage(buf ^ 1);
         __syncthreads();
     }
-    if constexpr (LONG && !Row::MIN) {
+    if constexpr (LONG) {
 #pragma unroll
         for (int m = 0; m < NT; m++) r[m] += tot[m];
     }

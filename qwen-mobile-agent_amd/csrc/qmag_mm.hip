@@ -17,14 +17,20 @@ namespace qmag {
 // super-blocks w, w + W, ... of the 16 rows against all its tokens, reading
 // the activations straight from memory (the workgroup's waves share none),
 // and the W partial results are added through LDS.
-template <int WT, int MT>
+//
+// Chains of eight super-blocks per wave and sum (n_in 32,768 over 8 waves and
+// 262,144 over 8, against 64 bits: Q4_K 1.06e-7 and 2.22e-7 in one sum, 9.7e-8
+// and 1.18e-7 in chains, the matvec's lane tree 1.39e-7 and 1.91e-7; Q6_K
+// 9.5e-8 and 2.05e-7, 8.3e-8 and 1.06e-7, tree 8.9e-8 and 1.51e-7).
+constexpr int SPLIT_CHAIN = 8;
+template <int WT, int MT, bool LNG>            // LNG: long rows (put_partials)
 __global__ __launch_bounds__(512) void mm_split_kernel(const uint8_t *__restrict__ W, const int8_t *__restrict__ xq,
                                                        const float *__restrict__ xd,
                                                        const int16_t *__restrict__ xsum, float *__restrict__ out,
                                                        int nb, int n_out, int T)
 {
     using Row = WRow<WT, 4>;
-    // [waves]: a weight image each, then (the same bytes) [MT][4][64] partials
+    // an image per wave, and the partials (split_lds)
     extern __shared__ __align__(16) uint8_t s_dyn[];
     const int lane = lane_id(), lr = lane & 15, q = lane >> 4;
     const int wv = (int)(threadIdx.x >> 6), nw = (int)(blockDim.x >> 6);
@@ -35,6 +41,8 @@ __global__ __launch_bounds__(512) void mm_split_kernel(const uint8_t *__restrict
 #pragma unroll
     for (int m = 0; m < MT; m++) tok[m] = (size_t)min(t0 + 16 * m + lr, T - 1) * nb;
     float r[MT][4] = {};
+    float *s_part = (float *)(s_dyn + (LNG ? nw * img.BYTES : 0));
+    int done = 0;
     if (wv < nb) img.request_all(wv);          // wave-uniform
     for (int ib = wv; ib < nb; ib += nw) {
         v4i a[MT][4];
@@ -87,13 +95,11 @@ __global__ __launch_bounds__(512) void mm_split_kernel(const uint8_t *__restrict
                 if constexpr (Row::MIN) v = fmaf(-w.dmin(), mn[m][i], v);
                 r[m][i] = fmaf(xdi, v, r[m][i]);
             }
+        if constexpr (LNG)
+            if (++done % SPLIT_CHAIN == 0) put_partials<MT>(s_part, wv, r, done > SPLIT_CHAIN);
     }
     __syncthreads();                           // every wave is done with its image
-    float *s_part = (float *)s_dyn;
-#pragma unroll
-    for (int m = 0; m < MT; m++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) s_part[((wv * MT + m) * 4 + i) * 64 + lane] = r[m][i];
+    put_partials<MT>(s_part, wv, r, LNG);   // of long rows every wave has a whole chain there
     __syncthreads();
     for (int k = (int)threadIdx.x; k < MT * 256; k += (int)blockDim.x) {
         // the waves' partials pairwise (as accurate as the matvec's lane tree)
@@ -116,34 +122,52 @@ __global__ __launch_bounds__(512) void mm_split_kernel(const uint8_t *__restrict
 // part; two waves per SIMD overlap these only in part (2048 -> 8192 x 512
 // tokens: 25 us, MFMA busy 36% and VALU 65% of it; the token loop before took
 // 280).
+//
+// One launch takes up to MM_CHAIN super-blocks of the rows and adds to out
+// behind the first: sums of eight super-blocks, added up over any longer row,
+// would round more than the matvec's lane tree again (n_in 32,768 against 64
+// bits: Q6_K 9.8e-8, the tree 8.8e-8, in launches of 32 super-blocks 8.4e-8;
+// Q4_K, in one sum 2.13e-7, the tree 1.39e-7, in launches of 64 1.04e-7).
 constexpr int MMT = 64, MMR = 128;
+template <int WT>
+constexpr int MM_CHAIN = WT == QMAG_TYPE_Q4_K ? 64 : 32;
 
 template <int WT>
 __global__ __launch_bounds__(256, 2) void mm_tile_kernel(const uint8_t *__restrict__ W,
                                                          const int8_t *__restrict__ xq,
                                                          const float *__restrict__ xd,
                                                          const int16_t *__restrict__ xsum, float *__restrict__ out,
-                                                         int nb, int n_out, int T)
+                                                         int nb, int n_out, int T, int ib0)
 {
     using Img = WImage<WT, 32>;
     __shared__ __align__(16) TileLds<2> s_t;
     __shared__ __align__(16) uint8_t s_w[4 * Img::BYTES];
-    const int lane = lane_id(), lr = lane & 31, h = lane >> 5, wv = (int)(threadIdx.x >> 6);
+    const int lane = lane_id(), lr = lane & 31, h = lane >> 5;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));        // uniform, and known to be
     const int row0 = (int)blockIdx.x * MMR + 32 * wv, t0 = (int)blockIdx.y * MMT;
     Img img;
     img.init(s_w + wv * Img::BYTES, W, row0, n_out, nb);
-    img.request_all(0);
+    img.request_all(ib0);
     TileSrc<2> src;
-    src.init(xq, xd, xsum, nb, [&](int t) { return min(t0 + t, T - 1); });
+    const size_t b0 = (size_t)t0 * nb;
+    src.init(xq + b0 * QK_K, xd + b0, xsum + b0 * 16, nb, [&](int t) { return min(t, T - 1 - t0); });
     v16f r[2];
-    tile_products<WT, 2, true>(img, nb, src, s_t, r);
+    tile_products<WT, 2, true>(img, ib0, min(ib0 + MM_CHAIN<WT>, nb), src, s_t, r);
+    // result i of group m: token t0 + at(m, i), weight row row0 + lr
+    auto at = [&](int m, int i) { return 32 * m + 8 * (i >> 2) + 4 * h + (i & 3); };
+    float *o = out + (size_t)t0 * n_out + row0 + lr;
+    const int tn = row0 + lr < n_out ? T - t0 : 0;         // tokens to write
+    if (ib0)
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if (at(m, i) < tn) r[m][i] += o[(size_t)at(m, i) * n_out];
 #pragma unroll
     for (int m = 0; m < 2; m++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int t = t0 + 32 * m + 8 * (i >> 2) + 4 * h + (i & 3);
-            if (t < T && row0 + lr < n_out) out[(size_t)t * n_out + row0 + lr] = r[m][i];
-        }
+        for (int i = 0; i < 16; i++)
+            if (at(m, i) < tn) o[(size_t)at(m, i) * n_out] = r[m][i];
 }
 
 // ------------------------------------------------------------------- host --
@@ -166,21 +190,26 @@ static int launch_mm_t(const int8_t *xq, const float *xd, const int16_t *xsum, c
     const uint8_t *w = (const uint8_t *)W;
     const int rt = (n_out + MMR - 1) / MMR, tt = (T + MMT - 1) / MMT;
     if ((long)rt * tt >= (WT == QMAG_TYPE_Q4_K ? MM_TILES_Q4 : MM_TILES_Q6) && tt <= 65535) {
-        hipLaunchKernelGGL(mm_tile_kernel<WT>, dim3(rt, tt), dim3(256), 0, s, w, xq, xd, xsum, out, nb, n_out, T);
+        for (int ib0 = 0; ib0 < nb; ib0 += MM_CHAIN<WT>)
+            hipLaunchKernelGGL(mm_tile_kernel<WT>, dim3(rt, tt), dim3(256), 0, s, w, xq, xd, xsum, out, nb, n_out, T,
+                               ib0);
     } else {
         const int mt = T > 48 ? 4 : (T + 15) / 16;
         const dim3 grid((n_out + 15) / 16, (T + 16 * mt - 1) / (16 * mt));
         const int most = (long)grid.x * grid.y >= MM_SPLIT8_WGS ? 4 : 8;
         int nw = 1;
         while (nw < most && nw < nb) nw *= 2;
-        const size_t part = sizeof(float) * 256 * (size_t)mt, image = WImage<WT, 16>::BYTES;
-        const size_t lds = (size_t)nw * (part > image ? part : image);
+        const size_t lds = split_lds(nb, nw, SPLIT_CHAIN, mt, WImage<WT, 16>::BYTES);
         const dim3 wg(64 * nw);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, wg, lds, s, w, xq, xd, xsum, out, nb, n_out, T);
+        };
+        const bool lng = long_row(nb, nw, SPLIT_CHAIN);
         switch (mt) {
-        case 1: hipLaunchKernelGGL((mm_split_kernel<WT, 1>), grid, wg, lds, s, w, xq, xd, xsum, out, nb, n_out, T); break;
-        case 2: hipLaunchKernelGGL((mm_split_kernel<WT, 2>), grid, wg, lds, s, w, xq, xd, xsum, out, nb, n_out, T); break;
-        case 3: hipLaunchKernelGGL((mm_split_kernel<WT, 3>), grid, wg, lds, s, w, xq, xd, xsum, out, nb, n_out, T); break;
-        default: hipLaunchKernelGGL((mm_split_kernel<WT, 4>), grid, wg, lds, s, w, xq, xd, xsum, out, nb, n_out, T); break;
+        case 1: launch(lng ? mm_split_kernel<WT, 1, true> : mm_split_kernel<WT, 1, false>); break;
+        case 2: launch(lng ? mm_split_kernel<WT, 2, true> : mm_split_kernel<WT, 2, false>); break;
+        case 3: launch(lng ? mm_split_kernel<WT, 3, true> : mm_split_kernel<WT, 3, false>); break;
+        default: launch(lng ? mm_split_kernel<WT, 4, true> : mm_split_kernel<WT, 4, false>); break;
         }
     }
     QMAG_HIP(hipGetLastError());

@@ -151,6 +151,65 @@ def test_matmul_f32_several_tokens(qm, orc, wtype, n_in, n_out, T):
     assert max_rel_err(got, ref) < (12 + n_in / 2048) * 2.0 ** -24 * n_in ** 0.5
 
 
+def _deq64(raw, wtype, n_in):
+    """float64 weights of block bytes, without rounding: [rows, n_in]."""
+    b = raw.reshape(-1, 144 if wtype == 12 else 210)
+    n = b.shape[0]
+    f16 = lambda c: b[:, c:c + 2].copy().view(np.float16).astype(np.float64)
+    if wtype == 12:
+        s, m, z = b[:, 4:8], b[:, 8:12], b[:, 12:16]
+        sc = np.concatenate([s & 63, (z & 15) | ((s >> 6) << 4)], 1) * f16(0)
+        mn = np.concatenate([m & 63, (z >> 4) | ((m >> 6) << 4)], 1) * f16(2)
+        qs = b[:, 16:].reshape(n, 4, 32)
+        q = np.stack([qs & 15, qs >> 4], 2).reshape(n, 8, 32)
+        return (q * sc[:, :, None] - mn[:, :, None]).reshape(-1, n_in)
+    ql, qh = b[:, :128].reshape(n, 2, 2, 32), b[:, 128:192].reshape(n, 2, 32)
+    lo = np.concatenate([ql & 15, ql >> 4], 2)
+    q = lo | (np.stack([(qh >> (2 * k)) & 3 for k in range(4)], 2) << 4)
+    sc = b[:, 192:208].copy().view(np.int8) * f16(208)
+    return ((q.reshape(n, 16, 16) - 32.0) * sc[:, :, None]).reshape(-1, n_in)
+
+
+def _long_row_errors(qm, orc, call, quantised, wtype, n_in, n_out, T):
+    """Relative error (2-norm against 64 bits, over the last 250 rows of the last 8
+    tokens) of one call of T tokens and of the same tokens one by one."""
+    rng = np.random.default_rng(T + wtype)
+    W = _rand_blocks(rng, wtype, n_in * n_out // 256)
+    x = rng.standard_normal((T, n_in), dtype=np.float32)
+    Wd, xb, out, one = qm.DBuf.from_array(W), qm.DBuf.from_array(x), qm.DBuf(4 * T * n_out), qm.DBuf(4 * n_out)
+    call(xb, Wd, n_in, n_out, T, wtype, out)
+    got = out.download(np.float32).reshape(T, n_out)[-8:, -250:]
+    ones, xe = [], x[-8:].astype(np.float64)
+    for t in range(8):
+        call(qm.DBuf.from_array(x[T - 8 + t]), Wd, n_in, n_out, 1, wtype, one)
+        ones.append(one.download(np.float32)[-250:])
+        if quantised:
+            xq, xd, _ = orc.q8k_quant(x[T - 8 + t])
+            xe[t] = (xq.reshape(-1, 256) * xd.astype(np.float64)[:, None]).reshape(-1)
+    ref = xe @ _deq64(W[-250 * (W.size // n_out):], wtype, n_in).T
+    err = lambda v: float(np.linalg.norm(v - ref) / np.linalg.norm(ref))
+    return err(got), err(np.array(ones))
+
+
+@pytest.mark.parametrize("wtype", [12, 14])
+@pytest.mark.parametrize("n_in,n_out,T", [(16640, 250, 37), (65536, 256, 40), (5120, 1000, 893), (16640, 1000, 893),
+                                          (65536, 1024, 896)])
+def test_matmul_long_rows_error(qm, orc, wtype, n_in, n_out, T):
+    """20, 65 and 256 super-blocks per row on the split-K kernel (two shapes) and
+    the tile kernel.  Sums in chains of 8, those in chains of at most 8, those
+    in turn (nb / 64) or pairwise (3), each addition rounding by at most u =
+    2^-24 of a partial sum no larger than the result's order: below u sqrt(8 + 8
+    + nb / 64 + 3) in the 2-norm, about three times what is seen.  At 256
+    super-blocks also no further off than one token at a time (the matvec's
+    lane tree; 5%: two estimates over 2,000 results): in one running sum per
+    wave or row the tile kernel was 2.0 (Q4_K) and 1.18 (Q6_K) times as far
+    off, the split kernel 1.14 (Q6_K)."""
+    several, one = _long_row_errors(qm, orc, qm.matmul_dev, True, wtype, n_in, n_out, T)
+    nb = n_in // 256
+    assert several < 2.0 ** -24 * (19 + nb / 64) ** 0.5
+    assert nb < 256 or several < 1.05 * one
+
+
 @pytest.mark.parametrize("wtype", [12, 14])
 @pytest.mark.parametrize("at", [0, 8448, 130000])
 def test_matmul_f32_out_on_x(qm, orc, wtype, at):
