@@ -9,7 +9,8 @@
 // assignment of k to lanes serves as long as both operands use it.  The sums are
 // kept as accurate as the one-token kernel's lane tree: chains of 8 products
 // (two MFMAs), added pairwise within a super-block and over the waves (one
-// chain per step of 64 products gave 1.57e-7 of the result against 9.7e-8).
+// chain per step of 64 products gave 1.57e-7 of the result against 9.7e-8),
+// and over a long row in chains of super-blocks (mmf_chain).
 // What bounds it at 24 tokens x 2048 x 2048 (8.6 us with Q4_K rows, 9.6 with
 // Q6_K; the one-token kernel 13.4 and 20.8) is the round trips of a wave's super-block; requesting
 // x a step ahead cost more in registers (two waves per SIMD) than it hid: 10.1.
@@ -53,7 +54,13 @@ struct Deq16 {
     }
 };
 
-template <int WT, int MT>
+// Super-blocks of a wave per running sum: four, and eight once a wave has more
+// than 32 (Q4_K, against 64 bits, in one sum / in chains / the one-token
+// kernel: n_in 16,384 1.10e-7 / 1.07e-7 / 1.07e-7, 65,536 1.43e-7 / 1.17e-7 /
+// 1.17e-7, 262,144 2.28e-7 / 1.35e-7 / 1.51e-7; chains of eight at 16,384 1.10e-7).
+__host__ __device__ __forceinline__ int mmf_chain(int nb, int nw) { return nb > 32 * nw ? 8 : 4; }
+
+template <int WT, int MT, bool LNG>            // LNG: long rows (put_partials)
 __global__ __launch_bounds__(512) void mmf_kernel(const uint8_t *__restrict__ W, const float *__restrict__ x,
                                                   float *__restrict__ out, int nb, int n_out, int T)
 {
@@ -68,6 +75,9 @@ __global__ __launch_bounds__(512) void mmf_kernel(const uint8_t *__restrict__ W,
 #pragma unroll
     for (int m = 0; m < MT; m++) xp[m] = x + (size_t)min(t0 + 16 * m + lr, T - 1) * nb * QK_K;
     float r[MT][4] = {};
+    float *s_part = (float *)(s_dyn + (LNG ? nw * img.BYTES : 0));
+    const int chain = mmf_chain(nb, nw);
+    int done = 0;
     if (wv < nb) img.request_all(wv);          // wave-uniform
     for (int ib = wv; ib < nb; ib += nw) {
         img.store();
@@ -104,13 +114,11 @@ __global__ __launch_bounds__(512) void mmf_kernel(const uint8_t *__restrict__ W,
         for (int m = 0; m < MT; m++)
 #pragma unroll
             for (int i = 0; i < 4; i++) r[m][i] += (acc[m][0][i] + acc[m][1][i]) + (acc[m][2][i] + acc[m][3][i]);
+        if constexpr (LNG)
+            if (++done % chain == 0) put_partials<MT>(s_part, wv, r, done > chain);
     }
     __syncthreads();                           // every wave is done with its image
-    float *s_part = (float *)s_dyn;
-#pragma unroll
-    for (int m = 0; m < MT; m++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) s_part[((wv * MT + m) * 4 + i) * 64 + lane] = r[m][i];
+    put_partials<MT>(s_part, wv, r, LNG);   // of long rows every wave has a whole chain there
     __syncthreads();
     for (int k = (int)threadIdx.x; k < MT * 256; k += (int)blockDim.x) {
         float p[8];
@@ -129,11 +137,13 @@ static int launch_mmf_t(const float *x, const uint8_t *W, int nb, int n_out, int
     const int mt = T > 16 ? 2 : 1;
     int nw = 1;
     while (nw < 8 && nw < nb) nw *= 2;
-    const size_t part = sizeof(float) * 256 * (size_t)mt, image = WImage<WT, 16>::BYTES;
-    const size_t lds = (size_t)nw * (part > image ? part : image);
+    const int chain = mmf_chain(nb, nw);
+    const bool lng = long_row(nb, nw, chain);
+    const size_t lds = split_lds(nb, nw, chain, mt, WImage<WT, 16>::BYTES);
     const dim3 grid((n_out + 15) / 16, (T + 16 * mt - 1) / (16 * mt)), wg(64 * nw);
-    if (mt == 1) hipLaunchKernelGGL((mmf_kernel<WT, 1>), grid, wg, lds, s, W, x, out, nb, n_out, T);
-    else hipLaunchKernelGGL((mmf_kernel<WT, 2>), grid, wg, lds, s, W, x, out, nb, n_out, T);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, wg, lds, s, W, x, out, nb, n_out, T); };
+    if (mt == 1) launch(lng ? mmf_kernel<WT, 1, true> : mmf_kernel<WT, 1, false>);
+    else launch(lng ? mmf_kernel<WT, 2, true> : mmf_kernel<WT, 2, false>);
     QMAG_HIP(hipGetLastError());
     return QMAG_OK;
 }

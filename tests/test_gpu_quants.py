@@ -211,6 +211,19 @@ def test_matmul_long_rows_error(qm, orc, wtype, n_in, n_out, T):
 
 
 @pytest.mark.parametrize("wtype", [12, 14])
+@pytest.mark.parametrize("n_in,T", [(8448, 16), (65536, 16), (65536, 40), (66816, 37)])
+def test_matmul_f32_long_rows_error(qm, orc, wtype, n_in, T):
+    """The same of the fp32 matrix-core kernel (its additions within a
+    super-block are 5 levels and 2 in turn more): chains of four and (from 257
+    super-blocks) of eight.  One running sum per wave was 1.22 and 1.13 times as
+    far off at 65,536."""
+    several, one = _long_row_errors(qm, orc, qm.matmul_f32_dev, False, wtype, n_in, 1000, T)
+    nb = n_in // 256
+    assert several < 2.0 ** -24 * (26 + nb / 64) ** 0.5
+    assert nb < 256 or several < 1.05 * one
+
+
+@pytest.mark.parametrize("wtype", [12, 14])
 @pytest.mark.parametrize("at", [0, 8448, 130000])
 def test_matmul_f32_out_on_x(qm, orc, wtype, at):
     """Rows longer than one 8192-value chunk, several tokens, out on x (from
