@@ -195,8 +195,8 @@ int qmag_matmul_q8k_dev(const int8_t *xq, const float *xd, const int16_t *xsum,
                         const void *W, int n_in, int n_out, int T, int wtype, float *out);
 
 /* matmul seam, nn.c:307-345: quantise each x[t] once, then the matvec (for
-   T = 1 and n_in up to 32,768 a single launch: the matvec quantises x
-   itself, bit-identically).  n_in: any multiple of 256. */
+   T = 1 a single launch where that is faster: the matvec quantises x itself,
+   bit-identically).  n_in: any multiple of 256. */
 int qmag_matmul_dev(const float *x, const void *W, int n_in, int n_out, int T, int wtype,
                     float *out);
 

@@ -84,7 +84,7 @@ int launch_mm(const int8_t *xq, const float *xd, const int16_t *xsum, const void
               int wtype, float *out, hipStream_t s);
 // T = 1 with x in f32: the matvec quantises x to Q8_K itself (bit-identical);
 // available for the calls matvec_x_supported() accepts
-bool matvec_x_supported(int n_in, int n_out, const float *x, const float *out);
+bool matvec_x_supported(int n_in, int n_out, int wtype, const float *x, const float *out);
 int launch_repack_q6k(const void *src, void *dst, int n_in, int n_out, hipStream_t s);
 // up to QMAG_MV_GROUP_MAX matrices over one x at T = 1, one launch
 struct MvGroup {

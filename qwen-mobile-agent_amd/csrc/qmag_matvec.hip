@@ -517,7 +517,8 @@ __global__ __launch_bounds__(256) void matvec_any_kernel(const uint8_t *__restri
 // Q8_K(x) into LDS as the tiled one-token kernel does, then runs the loop
 // above: the same bits.  Q6_K 5120 -> 1537: 5.5 us against 6.3, a launch of
 // about 2 us saved and Q8_K(x) computed beside the first rows' round trip.
-constexpr int MV_ANY_X_MAX_NB = 128;        // 37 KB of LDS
+// mv_any_x_pays says which calls take it.
+constexpr int MV_ANY_X_MAX_NB = 64;         // 18.7 KB of LDS; beyond, never the faster form
 template <int WT>
 __global__ __launch_bounds__(QMAG_MV_WG) void matvec_any_x_kernel(const uint8_t *__restrict__ W,
                                                                   const float *__restrict__ xf,
@@ -565,13 +566,19 @@ __global__ __launch_bounds__(QMAG_MV_WG) void matvec_any_x_kernel(const uint8_t 
     }
 }
 
+// a wave per row, at most 32 waves per CU
+static int n_cus() { return ctx().n_cu > 0 ? ctx().n_cu : 256; }
+static int mv_any_wgs(int n_out)
+{
+    const long cap = (long)n_cus() * 32, waves = n_out < cap ? n_out : cap;
+    return (int)((waves + 3) / 4);
+}
+
 template <int WT>
 static int launch_mv_any(const int8_t *xq, const float *xd, const int16_t *xsum, const void *W, int nb,
                          int n_out, int T, float *out, hipStream_t s, const float *xf)
 {
-    const long cap = (long)(ctx().n_cu > 0 ? ctx().n_cu : 256) * 32;    // waves
-    const long waves = n_out < cap ? n_out : cap;
-    const int wgs = (int)((waves + 3) / 4);
+    const int wgs = mv_any_wgs(n_out);
     prof_begin(PROF_MATVEC, s);
     if (xf)
         hipLaunchKernelGGL(matvec_any_x_kernel<WT>, dim3(wgs), dim3(QMAG_MV_WG), (size_t)nb * (QK_K + 32 + 4), s,
@@ -623,22 +630,44 @@ int launch_matvec(const int8_t *xq, const float *xd, const int16_t *xsum, const 
     return launch_mv_t<QMAG_TYPE_Q6_K_R>(xq, xd, xsum, W, n_in, n_out, T, out, s, nullptr);
 }
 
+// Whether the one-launch form of a row length without a tiled kernel is the
+// faster one: every workgroup quantises all of x, 8 blocks a round, which pays
+// while a CU gets few workgroups and rounds, or where it is spread over several
+// rows per wave (they read Q8_K(x) from LDS then).  Two-step / one launch, us,
+// on 256 CUs:
+//   few workgroups  Q6_K 5120 -> 4096 8.6 / 8.2, 7168 -> 4096 10.1 / 10.2; 10,240
+//                   -> 2048 (repacked) 8.7 / 8.2, 12,288 8.8 / 9.3; 16,384 -> 1024
+//                   8.6 / 8.2, 24,576 -> 512 9.9 / 10.3; Q4_K 16,128 -> 1300 7.8 / 8.8
+//   in between      Q4_K 7168 -> 8192 9.9 / 13.9, 16,384 -> 8192 15.8 / 25.8; Q6_K
+//                   768 -> 16,384 8.9 / 9.9; but Q4_K 1536 -> 16,384 8.9 / 8.4
+//   rows per wave   Q4_K 7168 -> 24,576 (3) 20.9 / 21.6, -> 40,000 (5) 41.0 / 34.1;
+//                   Q6_K 3840 -> 24,576 19.7 / 18.1, 2304 15.7 / 15.8, 768 -> 40,960
+//                   17.7 / 18.1
+static bool mv_any_x_pays(int nb, int n_out, int wtype)
+{
+    const int cus = n_cus(), per_cu = (mv_any_wgs(n_out) + cus - 1) / cus, rows = n_out / (32 * cus);
+    if (nb > MV_ANY_X_MAX_NB) return false;
+    if (per_cu <= 5) return per_cu * nb <= 82;
+    if (wtype == QMAG_TYPE_Q4_K) return nb <= 6 || rows >= 5;
+    return rows >= 5 || (rows >= 3 && nb >= 10);
+}
+
 // x and out overlapping: the two-step path reads all of x first, so the row
 // lengths that took it before the one-launch form keep it
-bool matvec_x_supported(int n_in, int n_out, const float *x, const float *out)
+bool matvec_x_supported(int n_in, int n_out, int wtype, const float *x, const float *out)
 {
-    if (n_in <= 0 || n_in % QK_K) return false;
+    if (n_in <= 0 || n_in % QK_K || n_out <= 0) return false;
     if (tiled_nb(n_in / QK_K)) return true;
     const uintptr_t xa = (uintptr_t)x, oa = (uintptr_t)out;
-    const bool apart = xa + sizeof(float) * (size_t)n_in <= oa ||
-                       oa + sizeof(float) * (size_t)(n_out > 0 ? n_out : 0) <= xa;
-    return n_in / QK_K <= MV_ANY_X_MAX_NB && apart;
+    const bool apart = xa + sizeof(float) * (size_t)n_in <= oa || oa + sizeof(float) * (size_t)n_out <= xa;
+    return apart && mv_any_x_pays(n_in / QK_K, n_out, wtype);
 }
 
 int launch_matvec_x(const float *x, const void *W, int n_in, int n_out, int wtype, float *out, hipStream_t s)
 {
     if (n_in <= 0 || n_in % QK_K || n_out <= 0) return fail(QMAG_ERR_ARG, "matvec: n_in=%d n_out=%d", n_in, n_out);
-    if (!matvec_x_supported(n_in, n_out, x, out)) return fail(QMAG_ERR_ARG, "matvec: internal: n_in=%d has no fused Q8_K form", n_in);
+    if (!tiled_nb(n_in / QK_K) && n_in / QK_K > MV_ANY_X_MAX_NB)
+        return fail(QMAG_ERR_ARG, "matvec: internal: n_in=%d has no fused Q8_K form", n_in);
     if (!x || !W || !out) return fail(QMAG_ERR_ARG, "matvec: null pointer");
     if (wtype == QMAG_TYPE_Q4_K)
         return launch_mv_t<QMAG_TYPE_Q4_K>(nullptr, nullptr, nullptr, W, n_in, n_out, 1, out, s, x);

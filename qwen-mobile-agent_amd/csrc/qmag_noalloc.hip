@@ -55,7 +55,8 @@ extern "C" int qmag_matmul_noalloc_dev(const float *x, const void *W, int n_in, 
     if (!sp) return fail(QMAG_ERR_NODEV, "matmul_noalloc: scratch address not set up");
     ProfSuspend quiet;        // per-kernel event timing allocates events: off here
     hipStream_t s = ctx().stream;
-    if (T == 1 && matvec_x_supported(n_in, n_out, x, out)) return launch_matvec_x(x, W, n_in, n_out, wtype, out, s);
+    if (T == 1 && matvec_x_supported(n_in, n_out, wtype, x, out))
+        return launch_matvec_x(x, W, n_in, n_out, wtype, out, s);
     int8_t *xq = (int8_t *)(sp + NA_XQ);
     float *xd = (float *)(sp + NA_XD);
     int16_t *xs = (int16_t *)(sp + NA_XS);

@@ -109,46 +109,39 @@ def test_q8k_dot_subnormal_scales(qm, orc):
         assert max_rel_err(out.download(np.float32), ref) < TOL
 
 
-@pytest.mark.parametrize("wtype", [12, 14])
-@pytest.mark.parametrize("n_in,n_out", [(768, 1), (1280, 37), (2816, 1030), (5120, 9), (32512, 5), (33024, 3)])
-def test_matmul_one_launch_any_row_length(qm, orc, wtype, n_in, n_out):
-    """At T = 1 a row length that is no power of two runs as one launch too (up
-    to 32,768 values, beyond which Q8_K(x) is its own launch): the bits of the
-    two-step path."""
-    W = orc.quantize(orc.fill_normal(n_in + 7, n_in * n_out, 0.0, 0.02), wtype)
+@pytest.mark.parametrize("wtype,n_in,n_out,launches", [
+    (12, 768, 1, 1), (14, 768, 1, 1), (12, 1280, 37, 1), (14, 2816, 1030, 1), (12, 5120, 9, 1), (270, 6144, 37, 1),
+    # few workgroups per CU: the line at 82 blocks (a CU's workgroups x super-blocks), and at 64 super-blocks
+    (14, 5120, 4096, 1), (14, 5376, 4096, 2), (12, 10496, 2048, 1), (12, 10752, 2048, 2), (270, 10240, 2048, 1),
+    (12, 16384, 5, 1), (14, 16640, 5, 2), (12, 32512, 5, 2), (14, 33024, 3, 2),
+    # more: short Q4_K rows, then several rows per wave
+    (12, 1536, 5200, 1), (12, 2304, 5200, 2), (14, 1536, 5200, 2), (12, 2304, 40959, 2), (12, 2304, 40960, 1),
+    (14, 2304, 24576, 2), (14, 2560, 24576, 1), (14, 2560, 24575, 2)])
+def test_matmul_one_launch_any_row_length(qm, orc, wtype, n_in, n_out, launches):
+    """At T = 1 a row length that is no power of two runs as one launch where
+    that is faster than two, on both sides of each line (256 CUs): the bits of
+    the two-step path, which a call with out on x always takes."""
+    W = _rand_blocks(np.random.default_rng(n_in + n_out), 12 if wtype == 12 else 14, n_in // 256 * n_out)
     x = orc.fill_normal(n_in, n_in, 0.0, 1.0)
-    Wd, xb, out = qm.DBuf.from_array(W), qm.DBuf.from_array(x), qm.DBuf(4 * n_out)
-    qm.matmul_dev(xb, Wd, n_in, n_out, 1, wtype, out)
+    Wd, xb, out = qm.DBuf.from_array(W), qm.DBuf(4 * max(n_in, n_out)), qm.DBuf(4 * n_out)
+    xb.upload(x)
+    if wtype == 270:
+        qm.repack_q6k_dev(Wd, Wd, n_in, n_out)
+    qm.prof_enable(True)
+    try:
+        qm.matmul_dev(xb, Wd, n_in, n_out, 1, wtype, out)
+        assert qm.prof_read("q8k")[0] == launches - 1
+    finally:
+        qm.prof_enable(False)
     one = out.download(np.uint32)
     xq, xd, xs = qm.DBuf(n_in), qm.DBuf(n_in // 64), qm.DBuf(n_in // 8)
     qm.q8k_quant_dev(xb, n_in, 1, xq, xd, xs)
     qm.matmul_q8k_dev(xq, xd, xs, Wd, n_in, n_out, 1, wtype, out)
     assert np.array_equal(one, out.download(np.uint32))
-    if n_out <= n_in:                          # out on x itself: x is read whole first
-        qm.check(qm.lib().qmag_matmul_dev(xb.ptr, Wd.ptr, n_in, n_out, 1, wtype, xb.ptr))
-        assert np.array_equal(one, xb.download(np.uint32, n_out))
-    assert max_rel_err(one.view(np.float32), orc.matmul_q8k(x, W, n_in, n_out, 1, wtype)[0]) < 1e-4
-
-
-@pytest.mark.parametrize("wtype", [12, 14])
-@pytest.mark.parametrize("n_in,n_out,T", [
-    # from the rule's line upwards: one and two tiles of 16 tokens per workgroup, rows and
-    # tokens off a tile, 1 to 8 waves with one and several super-blocks each, two token blocks
-    (256, 8001, 2), (512, 1067, 15), (768, 1001, 16), (1280, 1889, 17), (2304, 971, 33), (8448, 667, 48)])
-def test_matmul_f32_several_tokens(qm, orc, wtype, n_in, n_out, T):
-    """The fp32 matrix-core kernel against float64 over the oracle's
-    dequantised weights: fp32 weights (one rounding) and sums of at most 8
-    products, then log2(n_in / 8) pairwise or per-wave additions: below
-    (12 + n_in / 2048) 2^-24 of the sum of the terms' magnitudes, itself below
-    sqrt(n_in) max|y|."""
-    W = orc.quantize(orc.fill_normal(31 + n_in, n_in * n_out, 0.0, 0.02), wtype)
-    x = orc.fill_normal(T, n_in * T, 0.0, 1.0)
-    Wd, xd, out = qm.DBuf.from_array(W), qm.DBuf.from_array(x), qm.DBuf(4 * T * n_out)
-    qm.matmul_f32_dev(xd, Wd, n_in, n_out, T, wtype, out)
-    got = out.download(np.float32).reshape(T, n_out)
-    deq = orc.dequant(W, wtype, n_in * n_out).astype(np.float64).reshape(n_out, n_in)
-    ref = x.astype(np.float64).reshape(T, n_in) @ deq.T
-    assert max_rel_err(got, ref) < (12 + n_in / 2048) * 2.0 ** -24 * n_in ** 0.5
+    qm.check(qm.lib().qmag_matmul_dev(xb.ptr, Wd.ptr, n_in, n_out, 1, wtype, xb.ptr))     # x is read whole first
+    assert np.array_equal(one, xb.download(np.uint32, n_out))
+    if n_in * n_out < 1 << 23:
+        assert max_rel_err(one.view(np.float32), orc.matmul_q8k(x, W, n_in, n_out, 1, 12 if wtype == 12 else 14)[0]) < 1e-4
 
 
 def _deq64(raw, wtype, n_in):
