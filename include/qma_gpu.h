@@ -157,7 +157,7 @@ int qmag_prof_read(int kernel_id, long *count, double *total_ms);
    default: equally fast, and visible to rocprofv3's kernel tracing. */
 #define QMAG_OPT_COOP 3
 /* QMAG_OPT_GROUPED (default 1): qmag_moe_ffn_dev with T >= 16 tokens (the
-   prefill form) runs the grouped expert GEMM: (token, slot) pairs bucketed
+   prefill form; of few, large experts from 8) runs the grouped expert GEMM: (token, slot) pairs bucketed
    by expert into chunks of up to 64, gate/up and down as int8 MFMA tiles of
    16 pairs, each expert's weights read once per chunk; 0 selects the
    launch sequence (same results within the fp32 tolerance), which smaller

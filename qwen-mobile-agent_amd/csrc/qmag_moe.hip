@@ -539,15 +539,31 @@ static void launch_f32_down(const qmag_moe_layer *L, const int *sel, const float
 
 static bool pow2_in(int v, int lo, int hi) { return v >= lo && v <= hi && (v & (v - 1)) == 0; }
 
-// Batches of at least this many tokens take the grouped expert GEMM
-// (qmag_prefill.hip) when QMAG_OPT_GROUPED is on; smaller ones the launch
-// sequence below, which reads an expert once per token that chose it but is
-// five short launches.  Grouped / sequence, us per layer, with a router bias
-// (uneven experts, the grouped form's better case): n_embd 2048, 256 experts,
-// top 8, Q6_K down: 8 tokens 56 / 43, 12 62 / 56, 16 66 / 67, 24 74 / 88; Q4_K
-// down: 16 60 / 57, 24 66 / 74; 4096, 128 experts: 12 57 / 50, 16 60 / 59, 24
-// 71 / 75; 1024, 64 experts, top 4: 16 36 / 28, 35 40 / 40.
-constexpr int GROUPED_MIN_T = 16;
+// Whether a batch takes the grouped expert GEMM (qmag_prefill.hip; with
+// QMAG_OPT_GROUPED on) or the launch sequence below.  The sequence is five
+// short launches and reads an expert once per token that chose it, the repeats
+// from cache (6.5 TB/s in all); the grouped form reads each chosen expert once,
+// at 3.6 TB/s with few pairs a chunk, and its launches cost about 15 us more.
+// From GROUPED_MIN_T tokens on it is always taken; from GROUPED_FEW_T on where
+// those figures, with the experts that even routing chooses, favour it.  Grouped
+// / sequence, us per layer: 256 experts of n_embd 2048, n_ff 512, top 8: 8
+// tokens 58 / 40, 15 77 / 61; 16 experts, top 4: 15 38 / 35; 4096, 1024, 8
+// experts, top 8: 8 54 / 84, 15 54 / 137; 16 experts: 8 72 / 89, 15 73 / 146;
+// 4096, 512, 128 experts, top 8: 15 111 / 99.  Over 180 such points the choice
+// costs at most 9% (bias: fewer experts chosen) and 0.2% on average.
+constexpr int GROUPED_FEW_T = 8, GROUPED_MIN_T = 16;
+
+static bool grouped_pays(const qmag_moe_layer *L, int T)
+{
+    if (T >= GROUPED_MIN_T) return true;
+    if (T < GROUPED_FEW_T) return false;
+    const int db = L->t_down_exps == QMAG_TYPE_Q6_K ? Q6K_BYTES : Q4K_BYTES;
+    const double expert_mb = 1e-6 * L->n_ff * (L->n_embd / QK_K) * (2 * Q4K_BYTES + db);
+    double missed = 1.0;                       // share of the experts that no token chooses
+    for (int t = 0; t < T; t++) missed *= 1.0 - (double)L->n_used / L->n_expert;
+    const double chosen = L->n_expert * (1.0 - missed);
+    return expert_mb * (T * (L->n_used + 1) / 6.5 - (chosen + 1.0) / 3.6) > 15.0;
+}
 
 int moe_check_layer(const qmag_moe_layer *L, bool need_exps)
 {
@@ -706,7 +722,7 @@ int moe_ffn(const qmag_moe_layer *L, const float *x, float *out, int T, const fl
     st = moe_ws(L, T, ws);
     if (st) return st;
     const int K = L->n_used;
-    const bool grouped = T >= GROUPED_MIN_T && option(QMAG_OPT_GROUPED);
+    const bool grouped = option(QMAG_OPT_GROUPED) && grouped_pays(L, T);
     st = route_tokens(L, x, T, grouped, ws, s);
     if (st) return st;
     if (grouped) {

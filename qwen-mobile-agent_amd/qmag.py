@@ -167,8 +167,8 @@ OPT_GROUPED = 4
 
 
 def set_grouped(on: bool) -> None:
-    """Batches of >= 16 tokens: the grouped int8-MFMA expert GEMM (default) or
-    the launch sequence."""
+    """Batches of >= 16 tokens (of few, large experts >= 8): the grouped
+    int8-MFMA expert GEMM (default) or the launch sequence."""
     check(lib().qmag_set_option(OPT_GROUPED, 1 if on else 0))
 
 

@@ -105,6 +105,38 @@ def check_layer(qm, orc, rl, hl, x, T, run=None):
     return got
 
 
+def grouped_calls(qm, fn):
+    """fn()'s result and how many of its MoE calls took the grouped GEMM."""
+    qm.prof_enable(True)
+    try:
+        r = fn()
+        return r, qm.prof_read("group")[0]
+    finally:
+        qm.prof_enable(False)
+
+
+@pytest.mark.parametrize("cfg,T,grouped", [
+    (dict(n_embd=4096, n_ff=1024, n_expert=8, n_used=8, t_down=14), 7, 0),
+    (dict(n_embd=4096, n_ff=1024, n_expert=8, n_used=8, t_down=14), 8, 1),
+    (dict(n_embd=4096, n_ff=1024, n_expert=16, n_used=8, t_down=12), 9, 1),
+    (dict(n_embd=2048, n_ff=512, n_expert=256, n_used=8, t_down=14), 15, 0),
+])
+def test_moe_small_batch_path(qm, orc, cfg, T, grouped):
+    """8 to 15 tokens of few, large experts take the grouped GEMM (each expert
+    read once, not once per token), other batches below 16 the launch
+    sequence; the result against the oracle either way."""
+    rl = qm.ResidentLayer(seed=61, layer=0, **cfg)
+    hl = host_of(orc, rl)
+    x = orc.fill_normal(620 + T, T * cfg["n_embd"], 0.0, 1.0)
+    orc.set_threads(8)
+    try:
+        _, n = grouped_calls(qm, lambda: check_layer_staged(qm, orc, rl, hl, x, T, stage1_tokens=(0, T - 1)))
+    finally:
+        orc.set_threads(1)
+    assert n == grouped
+    rl.close()
+
+
 @pytest.mark.parametrize("cfg", [
     dict(n_embd=512, n_ff=256, n_expert=16, n_used=4, t_down=14),
     dict(n_embd=256, n_ff=512, n_expert=12, n_used=8, t_down=12),
