@@ -148,16 +148,23 @@ static int launch_mmf_t(const float *x, const uint8_t *W, int nb, int n_out, int
     return QMAG_OK;
 }
 
-// The one-token kernel spreads over the tokens and takes few rows faster; its
-// time grows with rows x tokens, this one's with a wave's super-blocks and
-// tiles.  That kernel / this one, us: Q4_K 2048 x 2048 x 4 tokens 4.2 / 5.4, x
-// 8 5.8 / 5.5, x 24 13.4 / 8.6; n_in 4096, 100 rows x 48 5.0 / 16.9, 4096 rows
-// x 2 6.8 / 8.7, x 4 10.2 / 9.1; Q6_K 2048 x 2048 x 4 5.1 / 6.3, x 8 8.1 / 6.4;
-// 4096, 4096 rows x 2 9.5 / 11.3, x 4 14.1 / 11.5.
+// The one-token kernel spreads over the tokens and takes few rows and tokens
+// faster; its time grows with rows x tokens x super-blocks, this one's with a
+// wave's super-blocks and tiles, of 32 tokens from 17 on, and fewer than five
+// super-blocks leave waves without work.  The line was fitted to 210 points a
+// type (1 to 16 super-blocks, 2 to 48 tokens, 250 to 8000 rows; at most 9%
+// (Q4_K) and 15% off the faster form, 0.2% on average).  That kernel / this
+// one, us: Q4_K n_in 256, 1000 rows x 48 3.5 / 6.5, 8000 x 16 5.5 / 4.9; 512,
+// 1000 x 32 3.6 / 6.1, 2000 x 48 7.5 / 6.2; 2048, 8000 x 2 5.7 / 8.3, 4000 x 3
+// 4.8 / 5.4, 8000 x 3 9.3 / 8.4, 16,000 x 3 15.0 / 15.2, 4000 x 4 5.7 / 5.5,
+// 2048 x 24 13.4 / 8.6; 4096, 100 x 48 5.0 / 16.9; Q6_K 512, 8000 x
+// 2 4.2 / 6.0, 2048, 4000 x 3 6.9 / 6.5, x 4 8.4 / 6.3, 16,000 x 2 15.2 / 18.8.
 bool mmf_supported(int nb, int n_out, int T, int wtype)
 {
-    const long least = wtype == QMAG_TYPE_Q4_K ? 16000 : 12000;
-    return T >= 2 && nb <= (1 << 18) && (long)n_out * T >= (T > 16 ? 2 : 1) * least;
+    const bool q4 = wtype == QMAG_TYPE_Q4_K;
+    if (T < (q4 ? 4 : 3) || nb > (1 << 18)) return false;
+    const double least = (q4 ? 14000 : 13000) * (T > 16 ? (q4 ? 2.0 : 1.6) : 1.0) * (nb < 5 ? 5.0 / nb : 1.0);
+    return (double)n_out * T >= least;
 }
 
 int launch_mmf(const float *x, const void *W, int nb, int n_out, int T, int wtype, float *out, hipStream_t s)
