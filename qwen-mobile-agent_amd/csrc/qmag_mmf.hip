@@ -154,8 +154,8 @@ static int launch_mmf_t(const float *x, const uint8_t *W, int nb, int n_out, int
 // super-blocks leave waves without work.  The line was fitted to 210 points a
 // type (1 to 16 super-blocks, 2 to 48 tokens, 250 to 8000 rows; at most 9%
 // (Q4_K) and 15% off the faster form, 0.2% on average).  That kernel / this
-// one, us: Q4_K n_in 256, 1000 rows x 48 3.5 / 6.5, 8000 x 16 5.5 / 4.9; 512,
-// 1000 x 32 3.6 / 6.1, 2000 x 48 7.5 / 6.2; 2048, 8000 x 2 5.7 / 8.3, 4000 x 3
+// one, us: Q4_K n_in 256, 1000 rows x 48 3.5 / 6.5, 8000 x 16 5.4 / 4.7; 512,
+// 1000 x 32 3.6 / 6.1, 2000 x 48 7.3 / 6.1; 2048, 8000 x 2 5.7 / 8.3, 4000 x 3
 // 4.8 / 5.4, 8000 x 3 9.3 / 8.4, 16,000 x 3 15.0 / 15.2, 4000 x 4 5.7 / 5.5,
 // 2048 x 24 13.4 / 8.6; 4096, 100 x 48 5.0 / 16.9; Q6_K 512, 8000 x
 // 2 4.2 / 6.0, 2048, 4000 x 3 6.9 / 6.5, x 4 8.4 / 6.3, 16,000 x 2 15.2 / 18.8.

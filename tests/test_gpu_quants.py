@@ -144,6 +144,27 @@ def test_matmul_one_launch_any_row_length(qm, orc, wtype, n_in, n_out, launches)
         assert max_rel_err(one.view(np.float32), orc.matmul_q8k(x, W, n_in, n_out, 1, 12 if wtype == 12 else 14)[0]) < 1e-4
 
 
+@pytest.mark.parametrize("wtype", [12, 14])
+@pytest.mark.parametrize("n_in,n_out,T", [
+    # from the rule's line upwards: one and two tiles of 16 tokens per workgroup, rows and
+    # tokens off a tile, 1 to 8 waves with one and several super-blocks each, two token blocks
+    (256, 17501, 4), (512, 2401, 15), (768, 1501, 16), (1280, 1889, 17), (2304, 971, 33), (8448, 667, 48)])
+def test_matmul_f32_several_tokens(qm, orc, wtype, n_in, n_out, T):
+    """The fp32 matrix-core kernel against float64 over the oracle's
+    dequantised weights: fp32 weights (one rounding) and sums of at most 8
+    products, then log2(n_in / 8) pairwise or per-wave additions: below
+    (12 + n_in / 2048) 2^-24 of the sum of the terms' magnitudes, itself below
+    sqrt(n_in) max|y|."""
+    W = orc.quantize(orc.fill_normal(31 + n_in, n_in * n_out, 0.0, 0.02), wtype)
+    x = orc.fill_normal(T, n_in * T, 0.0, 1.0)
+    Wd, xd, out = qm.DBuf.from_array(W), qm.DBuf.from_array(x), qm.DBuf(4 * T * n_out)
+    qm.matmul_f32_dev(xd, Wd, n_in, n_out, T, wtype, out)
+    got = out.download(np.float32).reshape(T, n_out)
+    deq = orc.dequant(W, wtype, n_in * n_out).astype(np.float64).reshape(n_out, n_in)
+    ref = x.astype(np.float64).reshape(T, n_in) @ deq.T
+    assert max_rel_err(got, ref) < (12 + n_in / 2048) * 2.0 ** -24 * n_in ** 0.5
+
+
 def _deq64(raw, wtype, n_in):
     """float64 weights of block bytes, without rounding: [rows, n_in]."""
     b = raw.reshape(-1, 144 if wtype == 12 else 210)
@@ -238,7 +259,8 @@ def test_matmul_f32_out_on_x(qm, orc, wtype, at):
 
 @pytest.mark.parametrize("wtype", [12, 14])
 @pytest.mark.parametrize("n_in,n_out,T", [(256, 100, 1), (2048, 512, 1), (512, 2048, 3), (8192, 64, 2),
-                                          (768, 77, 1), (12288, 40, 3), (16640, 33, 2), (24576, 17, 1)])
+                                          (768, 77, 1), (12288, 40, 3), (16640, 33, 2), (24576, 17, 1),
+                                          (256, 8001, 2), (512, 1067, 15), (768, 1001, 16)])
 def test_matmul_f32_dev(qm, orc, wtype, n_in, n_out, T):
     """The QMA_NOQ8K dequantise-then-dot path against the oracle's
     dot_q4_K_f32 / dot_q6_K_f32 per row (quants.c:80-133), including rows
