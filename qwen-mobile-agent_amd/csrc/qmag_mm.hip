@@ -171,12 +171,16 @@ __global__ __launch_bounds__(256, 2) void mm_tile_kernel(const uint8_t *__restri
 }
 
 // ------------------------------------------------------------------- host --
-// The split kernel fills the chip with few tiles, the tile kernel shares the
-// activations and builds each weight operand for 64 tokens instead of 16 MT
-// per wave.  Measured around the lines drawn here (n_in 2048, us per call with
-// the quantisation, split / tile): Q4_K 32 tiles 9.2 / 16.4, 64 tiles 18.2 /
-// 17.6, 128 tiles 30 / 17.9, 512 tiles 99 / 30.8; Q6_K 64 tiles 17.3 / 23.4,
-// 128 tiles 28 / 23.7, 512 tiles 94 / 38.
+// The split kernel's time grows with rows x tokens (in steps of 16 tokens); the
+// tile kernel builds each weight operand once for 64 tokens, however many there
+// are.  So it takes over from MM_TILES tiles on, counted by their tokens where
+// there is one row of tiles, and never at 16 tokens or fewer.  Split / tile, us with the quantisation: Q4_K
+// 2048 -> 8192 x 64 tokens 17.5 / 17.3 (the line), 16,384 x 32 17.7 / 17.6, x
+// 9 9.2 / 17.3, 151,936 x 4 44 / 64, x 16 67 / 65, x 24 96 / 67; 4096 -> 16,384
+// x 32 28.6 / 29.4, x 48 39.8 / 29.7; Q6_K 2048 -> 16,384 x 48 22.5 / 22.9, x
+// 64 28.0 / 23.2, 49,152 x 16 25.7 / 33.3, x 24 36.5 / 33.5; 8192 -> 16,384 x 48
+// 72.3 / 72.4; more than 64 tokens: Q4_K 2048 -> 6000 x 70 18.5 / 17.1, 4096 x 100
+// 15.6 / 17.0, 1000 x 460 20.4 / 18.3.
 constexpr long MM_TILES_Q4 = 64, MM_TILES_Q6 = 112;
 // Waves a row's super-blocks are split over: 8, and 4 once 512 workgroups
 // queue (151,936 rows x 4 tokens 44.5 against 49.9 us; 128 workgroups of 8,192
@@ -189,7 +193,9 @@ static int launch_mm_t(const int8_t *xq, const float *xd, const int16_t *xsum, c
 {
     const uint8_t *w = (const uint8_t *)W;
     const int rt = (n_out + MMR - 1) / MMR, tt = (T + MMT - 1) / MMT;
-    if ((long)rt * tt >= (WT == QMAG_TYPE_Q4_K ? MM_TILES_Q4 : MM_TILES_Q6) && tt <= 65535) {
+    const long tiles = WT == QMAG_TYPE_Q4_K ? MM_TILES_Q4 : MM_TILES_Q6;
+    const bool fill = tt > 1 ? (long)rt * tt >= tiles : T > 16 && (long)n_out * T >= tiles * MMR * MMT;
+    if (fill || n_out >= (1 << 27)) {          // a grid of the split kernel holds fewer rows
         for (int ib0 = 0; ib0 < nb; ib0 += MM_CHAIN<WT>)
             hipLaunchKernelGGL(mm_tile_kernel<WT>, dim3(rt, tt), dim3(256), 0, s, w, xq, xd, xsum, out, nb, n_out, T,
                                ib0);

@@ -249,9 +249,10 @@ def test_synth_weights_deterministic_and_scaled(qm, orc, wtype):
     # the split-K kernel: 1 to 4 tiles of 16 tokens, rows and tokens off a tile, fewer
     # super-blocks than waves, several per wave, 4 waves (512 workgroups) and 8
     (2048, 1, 9), (256, 15, 16), (2048, 33, 17), (4096, 16, 48), (2048, 100, 49), (6144, 17, 65), (1280, 70, 130),
-    (256, 8200, 20),
-    # the tile kernel (64 and 112 tiles of 128 rows x 64 tokens upwards), one to three super-blocks
-    (2048, 2049, 449), (256, 1793, 513), (768, 1921, 450)])
+    (256, 8200, 20), (512, 33000, 5), (512, 33000, 16), (256, 28000, 17),
+    # the tile kernel (from 64 and 112 tiles of 128 rows x 64 tokens, more than 16 tokens), one to three
+    # super-blocks; sums of eight added up apart, with four super-blocks left and none
+    (2048, 2049, 449), (256, 1793, 513), (768, 1921, 482), (5120, 1793, 513), (6144, 1793, 513), (256, 54001, 17)])
 def test_matmul_several_tokens(qm, orc, wtype, n_in, n_out, T):
     """The matrix-core kernels of the matmul seam against the oracle.  Their
     integer block sums are exact; per super-block and output three fp32
@@ -267,17 +268,22 @@ def test_matmul_several_tokens(qm, orc, wtype, n_in, n_out, T):
         qm.repack_q6k_dev(Wd, Wd, n_in, n_out)
     qm.matmul_dev(xd, Wd, n_in, n_out, T, wtype, out)
     got = out.download(np.float32).reshape(T, n_out)
-    ref = np.asarray(orc.matmul_q8k(x, W, n_in, n_out, T, 12 if wtype == 12 else 14)).reshape(T, n_out)
+    orc.set_threads(8)
+    try:
+        ref = np.asarray(orc.matmul_q8k(x, W, n_in, n_out, T, 12 if wtype == 12 else 14)).reshape(T, n_out)
+    finally:
+        orc.set_threads(1)
     nb = n_in // 256
     assert max_rel_err(got, ref) < (nb + 3) * 2.0 ** -24 * 4 * nb ** 0.5
 
 
+@pytest.mark.parametrize("n_out,T", [(50, 20), (1793, 513)])
 @pytest.mark.parametrize("off", [2, 4, 6])
-def test_matmul_several_tokens_row_offsets(qm, orc, off):
+def test_matmul_several_tokens_row_offsets(qm, orc, off, n_out, T):
     """Q6_K rows that start 2, 4 or 6 bytes past a 16-byte boundary: the weight
-    image reads a block from the dword it starts in, by its offset in the
-    matrix."""
-    n_in, n_out, T = 768, 50, 20
+    images of 16 rows (split-K kernel) and 32 (tile kernel) read a block from
+    the dword it starts in, by its offset in the matrix."""
+    n_in = 768
     W = orc.quantize(orc.fill_normal(8, n_in * n_out, 0.0, 0.02), 14)
     x = orc.fill_normal(9, n_in * T, 0.0, 1.0)
     Wd, xd, out = qm.DBuf(W.nbytes + 16), qm.DBuf.from_array(x), qm.DBuf(4 * T * n_out)

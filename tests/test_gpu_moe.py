@@ -441,27 +441,33 @@ def check_layer_staged(qm, orc, rl, hl, x, T, stage1_tokens=None, run=None):
     dict(n_embd=4096, n_ff=256, n_expert=16, n_used=4, t_down=14),
 ])
 def test_moe_grouped_small_shapes(qm, orc, cfg):
-    """Batches of >= 8 tokens run the grouped int8-MFMA expert GEMM; ragged
-    counts (37 tokens) leave partial 16-pair blocks in most buckets."""
+    """Batches of >= 16 tokens run the grouped int8-MFMA expert GEMM, 8 tokens of
+    these shapes the launch sequence; ragged counts (37 tokens) leave partial
+    16-pair blocks in most buckets."""
     hl = make_host_layer(orc, seed=13, **cfg)
     rl = qm.ResidentLayer.from_host(hl)
-    for T in (8, 37):
+    for T in (8, 16, 37):
         x = orc.fill_normal(300 + T, T * cfg["n_embd"], 0.0, 1.0)
-        check_layer_staged(qm, orc, rl, hl, x, T)
+        _, n = grouped_calls(qm, lambda: check_layer_staged(qm, orc, rl, hl, x, T))
+        assert n == (T >= 16)
     rl.close()
 
 
 def test_moe_grouped_sequence_option(qm, orc):
-    """QMAG_OPT_GROUPED = 0 sends a batch through the per-token launch
-    sequence, which is checked against the oracle the same way."""
+    """QMAG_OPT_GROUPED = 0 sends a batch that takes the grouped GEMM otherwise
+    through the launch sequence, which is checked against the oracle the same
+    way."""
     hl = make_host_layer(orc, seed=17, n_embd=512, n_ff=256, n_expert=16, n_used=4, t_down=14)
     rl = qm.ResidentLayer.from_host(hl)
-    x = orc.fill_normal(77, 12 * 512, 0.0, 1.0)
-    qm.set_grouped(False)
-    try:
-        check_layer_staged(qm, orc, rl, hl, x, 12)
-    finally:
-        qm.set_grouped(True)
+    T = 20
+    x = orc.fill_normal(77, T * 512, 0.0, 1.0)
+    for on in (False, True):
+        qm.set_grouped(on)
+        try:
+            _, n = grouped_calls(qm, lambda: check_layer_staged(qm, orc, rl, hl, x, T))
+        finally:
+            qm.set_grouped(True)
+        assert n == on
     rl.close()
 
 
