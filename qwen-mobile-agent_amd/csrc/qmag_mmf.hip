@@ -162,7 +162,8 @@ static int launch_mmf_t(const float *x, const uint8_t *W, int nb, int n_out, int
 bool mmf_supported(int nb, int n_out, int T, int wtype)
 {
     const bool q4 = wtype == QMAG_TYPE_Q4_K;
-    if (T < (q4 ? 4 : 3) || nb > (1 << 18)) return false;
+    // 32-bit offsets within 16 rows; 512 threads per 16 rows in one grid
+    if (T < (q4 ? 4 : 3) || nb > (1 << 18) || n_out >= (1 << 27)) return false;
     const double least = (q4 ? 14000 : 13000) * (T > 16 ? (q4 ? 2.0 : 1.6) : 1.0) * (nb < 5 ? 5.0 / nb : 1.0);
     return (double)n_out * T >= least;
 }

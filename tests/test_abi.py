@@ -101,6 +101,19 @@ def test_no_gpu_f32_entries_abort_with_a_message(built):
     assert "dot_q4_K_f32 called without a usable gfx950 device" in r.stderr
 
 
+def test_matrix_core_lines_stay_within_a_grid(built):
+    """A launch holds fewer than 2^32 threads in x: the fp32 matrix-core kernel
+    has a workgroup of up to 512 threads per 16 rows, so from 2^27 rows on the
+    one-token kernel (its grid is bounded) has to take the call."""
+    import ctypes as C
+    L = C.CDLL(built.LIB_PATH)
+    line = L["_ZN4qmag13mmf_supportedEiiii"]        # bool qmag::mmf_supported(nb, n_out, T, wtype)
+    line.restype = C.c_bool
+    for wtype in (12, 14):
+        assert line(8, (1 << 27) - 1, 4, wtype)
+        assert not line(8, 1 << 27, 4, wtype) and not line(1, (1 << 31) - 1, 65535, wtype)
+
+
 @pytest.mark.parametrize("lang", ["c", "c++"])
 def test_header_compiles_alone(lang, tmp_path):
     """qma_gpu.h is valid C99 and C++ on its own (an engine includes it from
