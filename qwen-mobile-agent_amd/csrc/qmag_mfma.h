@@ -329,13 +329,13 @@ inline size_t split_lds(int nb, int nw, int chain, int mt, int image)
 }
 
 // ------------------------------------------------------------------- tiles --
-// A workgroup of four waves: wave w holds 32 weight rows, all four share up to
-// 32 NT activation rows (tokens).  Per super-block those go through registers
+// A workgroup of four waves: wave w holds 32 weight rows, all four share 64
+// activation rows (tokens).  Per super-block those go through registers
 // into one of two LDS buffers while the other is consumed, and the wave's next
 // 32 weight blocks through registers into its image: one barrier per
 // super-block.
 constexpr int TILE_ROW = QK_K + 16;        // padded LDS row: 16 rows of a read start 4 banks apart
-template <int NT>
+constexpr int NT = 2;                      // 32-token groups of a tile
 struct TileLds {
     int8_t a[2][32 * NT * TILE_ROW];
     float d[2][32 * NT];
@@ -343,35 +343,34 @@ struct TileLds {
 };
 
 // The Q8_K rows a thread stages: 16-byte piece tid % 16 of tokens tid / 16 +
-// 16 k, the scale of token tid, half of the 16 sums of token tid / 2; row(t):
-// the row of the workgroup's token t, counted from the arrays' uniform bases.
+// 16 k, the scale of token tid, half of the 16 sums of token tid / 2 (tokens past
+// the last repeat it), from the uniform bases of the workgroup's first token.
 // The offsets are 32-bit (64 rows of at most 2^26 values): as pointers they
 // cost registers that the Q6_K loop does not have.
-template <int NT>
 struct TileSrc {
     const int8_t *xq;
     const float *xd;
     const int16_t *xs;
     uint32_t x[2 * NT], d, s;
-    template <class Row>
-    __device__ __forceinline__ void init(const int8_t *q, const float *scales, const int16_t *sums, int nb, Row row)
+    __device__ __forceinline__ void init(const int8_t *q, const float *scales, const int16_t *sums, int nb, int last)
     {
         const uint32_t tid = threadIdx.x;
+        auto row = [last](uint32_t t) { return (uint32_t)min((int)t, last); };
         xq = q;
         xd = scales;
         xs = sums;
 #pragma unroll
-        for (int k = 0; k < 2 * NT; k++) x[k] = (uint32_t)row((tid >> 4) + 16 * k) * (uint32_t)(nb * QK_K) + 16 * (tid & 15);
-        d = (uint32_t)row(tid & (32 * NT - 1)) * (uint32_t)nb;
-        s = (uint32_t)row((tid & (64 * NT - 1)) >> 1) * (uint32_t)(nb * 16) + 8 * (tid & 1);
+        for (int k = 0; k < 2 * NT; k++) x[k] = row((tid >> 4) + 16 * k) * (uint32_t)(nb * QK_K) + 16 * (tid & 15);
+        d = row(tid & (32 * NT - 1)) * (uint32_t)nb;
+        s = row((tid & (64 * NT - 1)) >> 1) * (uint32_t)(nb * 16) + 8 * (tid & 1);
     }
 };
 
 // r[m][i] of a lane: token 32 m + 8 (i / 4) + 4 (lane / 32) + i % 4, weight row
-// lane % 32, over the super-blocks ib0 .. nb - 1 (ib0 a multiple of eight).  LONG:
-// these may be more than eight.  The image's block ib0 has been requested.
-template <int WT, int NT, bool LONG, class Img>
-__device__ __forceinline__ void tile_products(Img &img, int ib0, int nb, const TileSrc<NT> &src, TileLds<NT> &lds,
+// lane % 32, over the super-blocks ib0 .. nb - 1 (ib0 a multiple of eight).  The
+// image's block ib0 has been requested.
+template <int WT, class Img>
+__device__ __forceinline__ void tile_products(Img &img, int ib0, int nb, const TileSrc &src, TileLds &lds,
                                               v16f (&r)[NT])
 {
     using Row = WRow<WT, 2>;
@@ -474,29 +473,25 @@ __device__ __forceinline__ void tile_products(Img &img, int ib0, int nb, const T
                     r[m][i] = fmaf(xv[k], v, r[m][i]);
                 }
             }
-        if constexpr (LONG) {
-            // sums of eight super-blocks are added up apart: one running sum
-            // over a long row would round more than the matvec's lane tree (n_in
-            // 8192: Q6_K 1.07e-7 of the result against 7.4e-8; Q4_K weights of
-            // random bytes 1.04e-7 against 8.5e-8, now 7.5e-8).  With its
-            // registers Q4_K of 4096 values and more takes 3% longer where a CU
-            // has one workgroup (4096 x 4096 x 256 30.2 -> 31.1 us).
-            if ((ib & 7) == 7 && ib + 1 < nb)
+        // sums of eight super-blocks are added up apart: one running sum
+        // over a long row would round more than the matvec's lane tree (n_in
+        // 8192: Q6_K 1.07e-7 of the result against 7.4e-8; Q4_K weights of
+        // random bytes 1.04e-7 against 8.5e-8, now 7.5e-8).  With its
+        // registers Q4_K of 4096 values and more takes 3% longer where a CU
+        // has one workgroup (4096 x 4096 x 256 30.2 -> 31.1 us).
+        if ((ib & 7) == 7 && ib + 1 < nb)
 #pragma unroll
-                for (int m = 0; m < NT; m++) {
-                    tot[m] += r[m];
+            for (int m = 0; m < NT; m++) {
+                tot[m] += r[m];
 #pragma unroll
-                    for (int i = 0; i < 16; i++) r[m][i] = 0.0f;
-                }
-        }
+                for (int i = 0; i < 16; i++) r[m][i] = 0.0f;
+            }
         img.store();
         stage(buf ^ 1);
         __syncthreads();
     }
-    if constexpr (LONG) {
 #pragma unroll
-        for (int m = 0; m < NT; m++) r[m] += tot[m];
-    }
+    for (int m = 0; m < NT; m++) r[m] += tot[m];
 }
 
 }  // namespace qmag

@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256, 2) void mm_tile_kernel(const uint8_t *__restri
                                                          int nb, int n_out, int T, int ib0)
 {
     using Img = WImage<WT, 32>;
-    __shared__ __align__(16) TileLds<2> s_t;
+    __shared__ __align__(16) TileLds s_t;
     __shared__ __align__(16) uint8_t s_w[4 * Img::BYTES];
     const int lane = lane_id(), lr = lane & 31, h = lane >> 5;
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));        // uniform, and known to be
@@ -148,23 +148,23 @@ __global__ __launch_bounds__(256, 2) void mm_tile_kernel(const uint8_t *__restri
     Img img;
     img.init(s_w + wv * Img::BYTES, W, row0, n_out, nb);
     img.request_all(ib0);
-    TileSrc<2> src;
+    TileSrc src;
     const size_t b0 = (size_t)t0 * nb;
-    src.init(xq + b0 * QK_K, xd + b0, xsum + b0 * 16, nb, [&](int t) { return min(t, T - 1 - t0); });
-    v16f r[2];
-    tile_products<WT, 2, true>(img, ib0, min(ib0 + MM_CHAIN<WT>, nb), src, s_t, r);
+    src.init(xq + b0 * QK_K, xd + b0, xsum + b0 * 16, nb, T - 1 - t0);
+    v16f r[NT];
+    tile_products<WT>(img, ib0, min(ib0 + MM_CHAIN<WT>, nb), src, s_t, r);
     // result i of group m: token t0 + at(m, i), weight row row0 + lr
     auto at = [&](int m, int i) { return 32 * m + 8 * (i >> 2) + 4 * h + (i & 3); };
     float *o = out + (size_t)t0 * n_out + row0 + lr;
     const int tn = row0 + lr < n_out ? T - t0 : 0;         // tokens to write
     if (ib0)
 #pragma unroll
-        for (int m = 0; m < 2; m++)
+        for (int m = 0; m < NT; m++)
 #pragma unroll
             for (int i = 0; i < 16; i++)
                 if (at(m, i) < tn) r[m][i] += o[(size_t)at(m, i) * n_out];
 #pragma unroll
-    for (int m = 0; m < 2; m++)
+    for (int m = 0; m < NT; m++)
 #pragma unroll
         for (int i = 0; i < 16; i++)
             if (at(m, i) < tn) o[(size_t)at(m, i) * n_out] = r[m][i];

@@ -26,7 +26,7 @@ struct Deq16 {
     using Row = WRow<WT, 4>;
     __device__ static __forceinline__ void weights(const Row &w, const typename Row::Raw &r, int s, float (&o)[16])
     {
-        const int half = (lane_id() >> 4) & 1, up = s & 1;
+        const int up = s & 1;
         if constexpr (WT == QMAG_TYPE_Q4_K) {
             const uint32_t byte = 8 * (2u * (uint32_t)(lane_id() >> 5) + (uint32_t)up);
             const uint32_t sc = ((w.S.sl[s >> 1] >> byte) & 7) | (((w.S.sh[s >> 1] >> byte) & 7) << 3);
@@ -43,7 +43,6 @@ struct Deq16 {
             const float ds = w.d() * (float)(int)(int8_t)(scw[s] >> (8 * (lane_id() >> 4)));
             const uint32_t l[4] = {r.l[0].x, r.l[0].y, r.l[0].z, r.l[0].w}, h[4] = {r.h.x, r.h.y, r.h.z, r.h.w};
             const uint32_t sh = 2u * (uint32_t)((lane_id() >> 5) + 2 * up);
-            (void)half;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const uint32_t q = ((up ? l[k] >> 4 : l[k]) & 0x0F0F0F0Fu) | (((h[k] >> sh) & 0x03030303u) << 4);

@@ -37,12 +37,9 @@
 // Every expert's weights are read once per 64-pair chunk (the shared
 // expert's by every chunk of 64 tokens); the pair buffers (h: T*S*F fp32,
 // y: T*S*N fp32) stay in HBM between kernels.
-#include "qmag_internal.h"
+#include "qmag_mfma.h"
 
 namespace qmag {
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int PB = 16;            // pairs per MFMA tile (the 16-wide M side)
 
@@ -364,12 +361,6 @@ __device__ __forceinline__ void q4w_mma(const Q4W<CH> &w, int c0, const int8_t *
 // 64 (q >> 1) + 16 (q & 1) + [0, 16), all of sub-block 4 half + 2 (q >> 1) +
 // hi.  Its scale bytes are per lane, and the activation operand is one
 // 16-byte LDS read at the same k.
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t mul_bytes(uint32_t q4, uint32_t m16)
-{
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, q4) * __builtin_bit_cast(u16x2, m16));
-}
-
 template <int CH>
 struct Q4V {
     uint4 hdr[CH], qa[CH], qb[CH];
@@ -438,10 +429,10 @@ __device__ __forceinline__ void q4v_mma_sp(const Q4V<CH> &w, const int8_t *aqA, 
             const uint32_t n3 = hi ? (src.w >> 4) & 0x0F0F0F0Fu : src.w & 0x0F0F0F0Fu;
             const uint32_t ml = __builtin_amdgcn_perm(0u, sl[half], hi ? sel1 : sel0);
             const uint32_t mh = __builtin_amdgcn_perm(0u, sh[half], hi ? sel1 : sel0);
-            const v4i B1 = {(int)mul_bytes(n0, ml), (int)mul_bytes(n1, ml), (int)mul_bytes(n2, ml),
-                            (int)mul_bytes(n3, ml)};
-            const v4i B2 = {(int)mul_bytes(n0, mh), (int)mul_bytes(n1, mh), (int)mul_bytes(n2, mh),
-                            (int)mul_bytes(n3, mh)};
+            const v4i B1 = {(int)pk_mul(n0, ml), (int)pk_mul(n1, ml), (int)pk_mul(n2, ml),
+                            (int)pk_mul(n3, ml)};
+            const v4i B2 = {(int)pk_mul(n0, mh), (int)pk_mul(n1, mh), (int)pk_mul(n2, mh),
+                            (int)pk_mul(n3, mh)};
             const int ko = c * QK_K + 128 * half + 32 * hi + koff;
             {
                 const v4i av = *(const v4i *)(aqA + lr * arow<NB>() + ko);

@@ -244,23 +244,24 @@ def test_synth_weights_deterministic_and_scaled(qm, orc, wtype):
     assert abs(w.std() - 0.02) < 0.002 and abs(w.mean()) < 0.002
 
 
-@pytest.mark.parametrize("wtype", [12, 14, 270])
-@pytest.mark.parametrize("n_in,n_out,T", [
+SEVERAL_TOKENS = [
     # the split-K kernel: 1 to 4 tiles of 16 tokens, rows and tokens off a tile, fewer
     # super-blocks than waves, several per wave, 4 waves (512 workgroups) and 8
     (2048, 1, 9), (256, 15, 16), (2048, 33, 17), (4096, 16, 48), (2048, 100, 49), (6144, 17, 65), (1280, 70, 130),
     (256, 8200, 20), (512, 33000, 5), (512, 33000, 16), (256, 28000, 17),
     # the tile kernel (from 64 and 112 tiles of 128 rows x 64 tokens, more than 16 tokens), one to three
     # super-blocks; sums of eight added up apart, with four super-blocks left and none
-    (2048, 2049, 449), (256, 1793, 513), (768, 1921, 482), (5120, 1793, 513), (6144, 1793, 513), (256, 54001, 17)])
+    (2048, 2049, 449), (256, 1793, 513), (768, 1921, 482), (5120, 1793, 513), (6144, 1793, 513), (256, 54001, 17)]
+
+
+@pytest.mark.parametrize("wtype,n_in,n_out,T", [(w, *s) for w in (12, 14, 270) for s in SEVERAL_TOKENS
+                                                if w != 270 or s[0] % 2048 == 0])     # repacked rows' lengths
 def test_matmul_several_tokens(qm, orc, wtype, n_in, n_out, T):
     """The matrix-core kernels of the matmul seam against the oracle.  Their
     integer block sums are exact; per super-block and output three fp32
     roundings, then the sum over the super-blocks (and waves): (nb + 3) 2^-24
     of the sum of the terms' magnitudes, which is below 4 sqrt(nb) max|y|
     here."""
-    if wtype == 270 and n_in % 2048:
-        pytest.skip("repacked rows need n_in % 2048 == 0")
     W = orc.quantize(orc.fill_normal(3 * n_in + n_out, n_in * n_out, 0.0, 0.02), 12 if wtype == 12 else 14)
     x = orc.fill_normal(T, n_in * T, 0.0, 1.0)
     Wd, xd, out = qm.DBuf.from_array(W), qm.DBuf.from_array(x), qm.DBuf(4 * T * n_out)
