@@ -102,9 +102,11 @@ template <int WT, int ROWS>
 struct WImage : WImageMap<WT, ROWS> {
     using M = WImageMap<WT, ROWS>;
     using M::BLOCK, M::BYTES, M::lead, M::NP, M::PIECES, M::Q4, M::REP, M::STRIDE, M::WP;
-    const uint8_t *base, *row;          // the wave's first row (uniform), the lane's row lane % ROWS
-    uint32_t at;                        // the first row's offset in the matrix (modulo 2^32)
-    int nb, src[WP], dst[WP];
+    const uint8_t *base;                // the dword that the wave's first row starts in (uniform)
+    uint32_t row;                       // from there, the lane's row lane % ROWS
+    int nb;
+    uint32_t src[WP];
+    int dst[WP];
     uint4 v[WP];
     uint32_t tail;
     uint8_t *img;
@@ -114,28 +116,27 @@ struct WImage : WImageMap<WT, ROWS> {
         img = lds;
         nb = nb_;
         const int first = M::row(0, row0, n_out), rb = nb * BLOCK;
-        base = W + (size_t)first * rb;
-        at = (uint32_t)first * (uint32_t)rb;
-        row = base + M::row_off(lane_id() % ROWS, row0, n_out, rb);
+        const uint32_t skew = M::skew(first, rb);
+        base = W + (size_t)first * rb - skew;
+        row = skew + (uint32_t)M::row_off(lane_id() % ROWS, row0, n_out, rb);
 #pragma unroll
         for (int k = 0; k < WP; k++) {
             const int p = M::piece(lane_id(), k), r = p / PIECES, j = p % PIECES;
             const int rel = M::row_off(r, row0, n_out, rb);
             dst[k] = M::dst(r, j);
-            src[k] = rel + M::src(j, nb);
+            src[k] = skew + (uint32_t)(rel + M::src(j, nb));
         }
     }
     __device__ __forceinline__ void request(int k, int ib)
     {
-        const uint32_t o = (uint32_t)src[k] + (uint32_t)ib * M::step(M::piece(lane_id(), k) % PIECES);
-        v[k] = ld16(base + (o - (uint32_t)lead(at + o)));
+        v[k] = ld16(base + M::from(src[k], ib, M::piece(lane_id(), k) % PIECES));
     }
     __device__ __forceinline__ void request_tail(int ib)
     {
         if constexpr (Q4) return;
-        const uint8_t *t = row + ib * M::tail_step() + M::tail0(nb);
-        if constexpr (REP) tail = ld2(t);
-        else tail = ld2(t - lead(at + (uint32_t)(row - base) + (uint32_t)ib * BLOCK)) | (ld2(t) << 16);
+        const uint32_t t = row + (uint32_t)(ib * M::tail_step() + M::tail0(nb));
+        if constexpr (REP) tail = ld2(base + t);
+        else tail = ld2(base + (t - lead(t))) | (ld2(base + t) << 16);
     }
     __device__ __forceinline__ void request_all(int ib)
     {
@@ -158,7 +159,7 @@ struct WImage : WImageMap<WT, ROWS> {
     __device__ __forceinline__ uint32_t shift(int ib) const
     {
         if constexpr (WT != QMAG_TYPE_Q6_K) return 0;
-        return 8 * (uint32_t)lead(at + (uint32_t)(row - base) + (uint32_t)ib * BLOCK);
+        return 8 * lead(row + (uint32_t)ib * BLOCK);
     }
 };
 

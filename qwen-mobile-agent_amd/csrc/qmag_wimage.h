@@ -41,9 +41,19 @@ struct WImageMap {
     }
     static constexpr uint32_t step(int j) { return REP ? (j < 12 ? 64u : 16u) : (uint32_t)BLOCK; }
     static constexpr int dst(int r, int j) { return r * STRIDE + 16 * j; }
-    // bytes between the dword a block starts in and the block, by its offset
-    // in the matrix (so that no read starts ahead of it)
-    static constexpr int lead(uint32_t off) { return WT == QMAG_TYPE_Q6_K ? (int)(off & 2) : 0; }
+    // A Q6_K block is read from the dword it starts in, `lead` bytes ahead of it.
+    // Offsets count from the dword that the wave's first row starts in, `skew`
+    // bytes ahead of that row (a row that starts inside a dword is not the
+    // matrix's first), so that no difference below is negative: counted from the
+    // row itself, a first row 2 bytes into a dword gave 2^32 - 2.
+    static constexpr uint32_t lead(uint32_t off) { return WT == QMAG_TYPE_Q6_K ? off & 2 : 0; }
+    static constexpr uint32_t skew(int row, int rb) { return lead((uint32_t)row * (uint32_t)rb); }
+    // where super-block ib's piece j is read from, start its block 0's offset
+    static constexpr uint32_t from(uint32_t start, int ib, int j)
+    {
+        const uint32_t o = start + (uint32_t)ib * step(j);
+        return o - lead(o);
+    }
     // the tail of super-block ib in its row (Q6_K formats)
     static constexpr int tail0(int nb) { return REP ? 208 * nb : 208; }
     static constexpr int tail_step() { return REP ? 2 : BLOCK; }

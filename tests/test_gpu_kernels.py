@@ -250,8 +250,9 @@ SEVERAL_TOKENS = [
     (2048, 1, 9), (256, 15, 16), (2048, 33, 17), (4096, 16, 48), (2048, 100, 49), (6144, 17, 65), (1280, 70, 130),
     (256, 8200, 20), (512, 33000, 5), (512, 33000, 16), (256, 28000, 17),
     # the tile kernel (from 64 and 112 tiles of 128 rows x 64 tokens, more than 16 tokens), one to three
-    # super-blocks; sums of eight added up apart, with four super-blocks left and none
-    (2048, 2049, 449), (256, 1793, 513), (768, 1921, 482), (5120, 1793, 513), (6144, 1793, 513), (256, 54001, 17)]
+    # super-blocks; waves past an odd last row of an odd number of super-blocks (Q6_K rows 2 bytes into a
+    # dword); sums of eight added up apart, with four super-blocks left and none
+    (2048, 2049, 449), (256, 1793, 513), (768, 1921, 482), (768, 1922, 482), (5120, 1793, 513), (6144, 1793, 513), (256, 54001, 17)]
 
 
 @pytest.mark.parametrize("wtype,n_in,n_out,T", [(w, *s) for w in (12, 14, 270) for s in SEVERAL_TOKENS

@@ -30,19 +30,26 @@ static long walk(int nb, int n_out)
     };
     // row0 also past the last row: the surplus waves of a workgroup
     for (int row0 = 0; row0 < n_out + 4 * ROWS; row0 += ROWS) {
-        const long first = (long)M::row(0, row0, n_out) * rb;
+        const int fr = M::row(0, row0, n_out);
+        const uint32_t skew = M::skew(fr, rb);
+        const long base = (long)fr * rb - skew;                 // may not lie ahead of the matrix either
+        in(base, 1, "base", row0, 0, 0, 0);
         for (int ib = 0; ib < nb; ib++)
             for (int lane = 0; lane < 64; lane++) {
                 for (int k = 0; k < M::WP; k++) {
                     const int p = M::piece(lane, k), r = p / M::PIECES, j = p % M::PIECES;
-                    const uint32_t o = (uint32_t)(M::row_off(r, row0, n_out, rb) + M::src(j, nb)) +
-                                       (uint32_t)ib * M::step(j);
-                    in(first + o - M::lead((uint32_t)first + o), 16, "piece", row0, lane, k, ib);
+                    const long block = M::row(r, row0, n_out) * (long)rb + ib * (long)M::BLOCK;
+                    const uint32_t o = M::from(skew + (uint32_t)(M::row_off(r, row0, n_out, rb) + M::src(j, nb)), ib, j);
+                    in(base + (long)o, 16, "piece", row0, lane, k, ib);
+                    if (!M::REP && base + (long)o != block + 16 * j - (long)M::lead((uint32_t)block) && !bad++)
+                        printf("%d rows %d nb %d n_out %d: piece %d of row0 %d block %d from %ld\n", WT, ROWS, nb, n_out, p,
+                               row0, ib, base + (long)o);
                 }
                 if (M::Q4) continue;
-                const long t = M::row_off(lane % ROWS, row0, n_out, rb) + M::tail0(nb) + ib * M::tail_step();
-                in(first + t - M::lead((uint32_t)(first + t)), 2, "tail", row0, lane, 0, ib);
-                in(first + t, 2, "tail", row0, lane, 0, ib);
+                const uint32_t t = skew + (uint32_t)M::row_off(lane % ROWS, row0, n_out, rb) +
+                                   (uint32_t)(M::tail0(nb) + ib * M::tail_step());
+                in(base + (long)(uint32_t)(t - M::lead(t)), 2, "tail", row0, lane, 0, ib);
+                in(base + (long)t, 2, "tail", row0, lane, 0, ib);
             }
     }
     return bad;
@@ -65,7 +72,8 @@ int main(int argc, char **argv)
 
 def test_every_request_lies_in_the_matrix(tmp_path):
     """All three layouts, images of 16 and 32 rows, one row, rows off a tile
-    and whole tiles, one to 128 super-blocks."""
+    and whole tiles, one to 128 super-blocks, in the kernels' own 32-bit
+    arithmetic; and a block's pieces are the block's."""
     cxx = shutil.which("g++")
     if not cxx:
         pytest.skip("no host compiler")
