@@ -117,11 +117,11 @@ __global__ __launch_bounds__(512) void mm_split_kernel(const uint8_t *__restrict
 // grid: rows / 128 x tokens / 64, rows fastest: workgroup i runs on XCD i % 8,
 // so each XCD's L2 holds an eighth of the weight rows and every token block
 // finds them there.  What bounds it is instruction issue: per 32 rows x 64
-// tokens x super-block 34 MFMAs (1,100 cycles) and 360 (Q4_K) or 600 (Q6_K)
+// tokens x super-block 34 MFMAs (1,100 cycles) and 390 (Q4_K) or 600 (Q6_K)
 // VALU instructions, a third of them the operands, most of the rest the fp32
 // part; two waves per SIMD overlap these only in part (2048 -> 8192 x 512
-// tokens: 25 us, MFMA busy 36% and VALU 65% of it; the token loop before took
-// 280).
+// tokens: 28.4 us, MFMA busy 39% and VALU 60% of the waves' time; the token
+// loop before took 280).
 //
 // One launch takes up to MM_CHAIN super-blocks of the rows and adds to out
 // behind the first: sums of eight super-blocks, added up over any longer row,
@@ -226,7 +226,8 @@ static int launch_mm_t(const int8_t *xq, const float *xd, const int16_t *xsum, c
 // loop over the tokens): Q4_K at 3 tokens 9.6 against 9.3 us (16,384 rows) and
 // 8.2 against 8.4 (n_in 8192), at 4 59.9 against 44.5 (151,936 rows); Q6_K at
 // 3 10.5 against 11.4, at 6 13.5 against 11.4, and rows beyond 4096 values at
-// 5 9.4 against 11.8, at 12 14.1 against 11.9.  They also take what this path
+// 5 9.4 against 11.8, at 12 14.1 against 11.9.  One row is no different (2048
+// values: 4 tokens level, 64 35.3 against 10.2).  They also take what this path
 // does not: rows beyond 2^26 values (32-bit offsets within 32 rows) and more
 // tokens than a grid holds.
 bool mm_supported(int nb, int T, int wtype)
